@@ -482,7 +482,7 @@ struct pz_handle {
     bool use_graph = true;
     size_t lds_radial = 0, lds_mphase = 0, lds_build = 0, lds_start = 0, lds_inv = 0, lds_start_coll = 0, lds_fd = 0,
            lds_fd_loop = 0;
-    size_t lds_gj = 0; // k_build_coll: blocked Gauss-Jordan panels
+    size_t lds_gj = 0; // k_build_coll: Gauss-Jordan panels
     bool mcoll_l2 = false; // collocation m-loop reads radial rows and tables through L2
     bool radial_big = false; // k_radial_loop_big for long azimuthal grids
     bool radial_inplace = false; // k_gather_r + k_radial_loop_inplace instead
@@ -1189,8 +1189,8 @@ static void setup(pz_handle *h)
         }
         d.PC_inv = h->dalloc<cd>((size_t)nm * N * 2 * N);
         d.U_inv = h->dalloc<double>((size_t)N * d.ldi);
-        // Gauss-Jordan blocks per m: T and xi (N x 2N real), psi (2N x 4N complex)
-        d.coll_ws = (2 * (size_t)N * 2 * N * sizeof(double) + (size_t)2 * N * 4 * N * sizeof(cd) + 255) & ~(size_t)255;
+        // Gauss-Jordan blocks per m: T and xi (N x N real), psi (2N x 2N complex)
+        d.coll_ws = (2 * (size_t)N * N * sizeof(double) + (size_t)2 * N * 2 * N * sizeof(cd) + 255) & ~(size_t)255;
         d.coll_work = h->dalloc<char>((size_t)nm * d.coll_ws);
         if (h->sch.l_assembly) {
             // boundary first-derivative rows for robin_bc (chebyshev.f90:338-360):
@@ -1231,11 +1231,8 @@ static void setup(pz_handle *h)
     hipDeviceProp_t prop;
     HIPCHK(hipGetDeviceProperties(&prop, dev));
     size_t lim = prop.sharedMemPerBlock;
-    // rebuild panels of 16 pivots where they fit next to the larger static LDS
-    // of the single-run and batched rebuild kernels, else 8
     const size_t gj_static = gj_static_lds();
-    d.gj_b = gj_lds_bytes<cd>(2 * N, 16) + gj_static <= lim ? 16 : 8;
-    h->lds_gj = gj_lds_bytes<cd>(2 * N, d.gj_b);
+    h->lds_gj = std::max(gj_lds_bytes<cd>(2 * N), (size_t)1024 * sizeof(double));
     if (d.coll && h->lds_mphase > lim) {
         h->mcoll_l2 = true;
         h->lds_mphase = MpLayout(N, h->mthreads, false).total;
@@ -1818,7 +1815,7 @@ extern "C" int pz_start(pz_handle *h)
             if (h->d.l_assembly) {
                 if (!h->d.A_inv || !h->d.dr_top || !h->d.dr_bot)
                     throw std::logic_error("assembly stage without its matrices");
-                hipLaunchKernelGGL(k_build_ass, dim3(h->nm), dim3(1024), 0, h->stream, h->d);
+                hipLaunchKernelGGL(k_build_ass, dim3(h->nm), dim3(1024), gj_lds_bytes<double>(h->N), h->stream, h->d);
             }
         } else {
             if (!h->d.T_RHSE2 || !h->d.T_RHSI || !h->d.P_RHSI)

@@ -16,42 +16,34 @@
 // Gauss-Jordan into A_inv [m][col][ldi].  grid (n_m), built once.
 __global__ void __launch_bounds__(1024) k_build_ass(const PzDev p __attribute__((grid_constant)))
 {
-    __shared__ double fcol[2 * 257];
+    extern __shared__ double2 gj_smem[]; // gj_lds_bytes<double>(n_r) bytes
     const int mi = blockIdx.x, N = p.N, m = p.idx2m[mi], tid = threadIdx.x, nc = p.ncheb, ldi = p.ldi;
     if (m == 0) return;
     const RadView R(p.radc, N);
-    double *W = (double *)(p.coll_work + (size_t)mi * p.coll_ws); // N x 2N, row-major
+    double *W = (double *)(p.coll_work + (size_t)mi * p.coll_ws); // N x N, row-major
     const double rn = p.rnorm, dm2 = (double)m * (double)m;
-    for (int t = tid; t < N * 2 * N; t += blockDim.x) {
-        const int r = t / (2 * N), c = t - r * 2 * N;
+    for (int t = tid; t < N * N; t += blockDim.x) {
+        const int r = t / N, c = t - r * N;
         double a;
-        if (c >= N) {
-            a = (c - N == r) ? 1.0 : 0.0;
-        } else {
-            const bool in = c < nc;
-            if (r == 0) a = in ? rn * PZ_CM(0, c) : 0.0;
-            else if (r == N - 1) a = in ? rn * PZ_CM(N - 1, c) : 0.0;
-            else if (r == 1) a = !in ? 0.0 : (p.ktopv == 1 ? rn * (PZ_CD2M(0, c) - R.or1(0) * PZ_CDM(0, c)) : rn * PZ_CDM(0, c));
-            else if (r == N - 2)
-                a = !in ? 0.0
-                        : (p.kbotv == 1 ? rn * (PZ_CD2M(N - 1, c) - R.or1(N - 1) * PZ_CDM(N - 1, c))
-                                        : rn * PZ_CDM(N - 1, c));
-            else
-                a = -rn * (PZ_CD2M(r, c) + (R.or1(r) + R.beta(r)) * PZ_CDM(r, c) +
-                           (R.or1(r) * R.beta(r) + R.dbeta(r) - dm2 * R.or2(r)) * PZ_CM(r, c));
-            if (c == 0 || c == N - 1) a *= p.boundary_fac;
-        }
+        const bool in = c < nc;
+        if (r == 0) a = in ? rn * PZ_CM(0, c) : 0.0;
+        else if (r == N - 1) a = in ? rn * PZ_CM(N - 1, c) : 0.0;
+        else if (r == 1) a = !in ? 0.0 : (p.ktopv == 1 ? rn * (PZ_CD2M(0, c) - R.or1(0) * PZ_CDM(0, c)) : rn * PZ_CDM(0, c));
+        else if (r == N - 2)
+            a = !in ? 0.0
+                    : (p.kbotv == 1 ? rn * (PZ_CD2M(N - 1, c) - R.or1(N - 1) * PZ_CDM(N - 1, c))
+                                    : rn * PZ_CDM(N - 1, c));
+        else
+            a = -rn * (PZ_CD2M(r, c) + (R.or1(r) + R.beta(r)) * PZ_CDM(r, c) +
+                       (R.or1(r) * R.beta(r) + R.dbeta(r) - dm2 * R.or2(r)) * PZ_CM(r, c));
+        if (c == 0 || c == N - 1) a *= p.boundary_fac;
         W[t] = a;
     }
     __syncthreads();
-    const int info = gj_invert<double>(W, N, fcol);
+    const int info = gj_invert<double>(W, N, N, (char *)gj_smem);
     if (tid == 0 && info) p.info[mi] = info; // reported as a singular matrix
     if (info) return;
-    double *out = p.A_inv + (size_t)mi * N * ldi;
-    for (int t = tid; t < N * ldi; t += blockDim.x) {
-        const int c = t / ldi, r = t - c * ldi;
-        out[(size_t)c * ldi + r] = r < N ? W[(size_t)r * 2 * N + N + c] : 0.0;
-    }
+    coll_store_inverse<double>(W, N, N, (char *)gj_smem, nullptr, nullptr, p.A_inv + (size_t)mi * N * ldi, ldi);
 }
 
 // old + sum_s b_exp(s) expl(s) + sum_s b_imp(s) impl(s) for element q

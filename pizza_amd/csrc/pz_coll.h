@@ -5,6 +5,7 @@
 // Included once by pz_api.hip, after pz_mphase.h.
 #pragma once
 #include "pz_mphase.h"
+#include "pz_gj.h"
 
 __device__ __forceinline__ double msub(double a, double b) { return a - b; }
 __device__ __forceinline__ cd msub(cd a, cd b) { return csub(a, b); }
@@ -12,235 +13,96 @@ __device__ __forceinline__ cd msub(cd a, cd b) { return csub(a, b); }
 __device__ __forceinline__ double mabs2(double a) { return fabs(a); }
 __device__ __forceinline__ double mabs2(cd a) { return hypot(a.x, a.y); }
 
-// ---------------------------------------------------------------------------
-// In-place Gauss-Jordan inversion with partial pivoting of the left half of
-// the row-major n x 2n block W = [A | I] by one workgroup; on return the
-// right half holds A^{-1}.  f: LDS scratch of n values.  Returns the
-// LAPACK-style info (k + 1 of the first zero pivot, 0 if none).
-// ---------------------------------------------------------------------------
-template <class M>
-__device__ int gj_invert(M *W, int n, M *f)
-{
-    __shared__ int s_p, s_info;
-    __shared__ double s_v[32];
-    __shared__ int s_i[32];
-    const int tid = threadIdx.x, nt = blockDim.x, w2 = 2 * n;
-    if (tid == 0) s_info = 0;
-    for (int t = tid; t < n * n; t += nt) {
-        const int i = t / n, j = t - i * n;
-        W[(size_t)i * w2 + n + j] = i == j ? mk_elem<M>(1.0, 0.0) : mzero<M>();
-    }
-    __syncthreads();
-    for (int k = 0; k < n; k++) {
-        // pivot: first row of the largest |re| + |im| in column k (i >= k)
-        double bv = -1.0;
-        int bi = n;
-        for (int i = k + tid; i < n; i += nt) {
-            const double v = mabs1(W[(size_t)i * w2 + k]);
-            if (v > bv) { bv = v; bi = i; }
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            const double ov = __shfl_xor(bv, o, 64);
-            const int oi = __shfl_xor(bi, o, 64);
-            if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-        }
-        if ((tid & 63) == 0) { s_v[tid >> 6] = bv; s_i[tid >> 6] = bi; }
-        __syncthreads();
-        if (tid == 0) {
-            double v = s_v[0];
-            int ii = s_i[0];
-            for (int q = 1; q < (nt + 63) / 64; q++)
-                if (s_v[q] > v || (s_v[q] == v && s_i[q] < ii)) { v = s_v[q]; ii = s_i[q]; }
-            s_p = ii;
-            if (!(v > 0.0) && s_info == 0) s_info = k + 1;
-        }
-        __syncthreads();
-        const int p = s_p;
-        if (s_info != 0) break;
-        if (p != k)
-            for (int j = k + tid; j < w2; j += nt) {
-                const M t = W[(size_t)k * w2 + j];
-                W[(size_t)k * w2 + j] = W[(size_t)p * w2 + j];
-                W[(size_t)p * w2 + j] = t;
-            }
-        __syncthreads();
-        const M rp = mrecip(W[(size_t)k * w2 + k]);
-        __syncthreads();
-        for (int j = k + tid; j < w2; j += nt) W[(size_t)k * w2 + j] = mmm(W[(size_t)k * w2 + j], rp);
-        for (int i = tid; i < n; i += nt) f[i] = i == k ? mzero<M>() : W[(size_t)i * w2 + k];
-        __syncthreads();
-        const int wj = w2 - k;
-        for (int t = tid; t < n * wj; t += nt) {
-            const int i = t / wj, j = k + (t - i * wj);
-            if (i != k) W[(size_t)i * w2 + j] = msub(W[(size_t)i * w2 + j], mmm(f[i], W[(size_t)k * w2 + j]));
-        }
-        __syncthreads();
-    }
-    __syncthreads();
-    return s_info;
-}
-
-#define GJ_BMAX 16 // widest panel (pivot columns per panel)
-#define GJ_CH 64   // columns per chunk of the panel update
-// dynamic LDS bytes of gj_invert_blk for n x n matrices of element M and
-// panels of B pivot columns
-template <class M>
-__host__ __device__ inline size_t gj_lds_bytes(int n, int B)
-{
-    return sizeof(M) * (2 * (size_t)n * B + (size_t)B * GJ_CH + 2 * (size_t)B);
-}
-
-// ---------------------------------------------------------------------------
-// Blocked Gauss-Jordan inversion with partial pivoting of the left half of
-// the row-major n x 2n block W = [A | I] by one workgroup, forming only the
-// first nr columns of A^{-1} in W's right half.  Each panel of B pivot
-// columns is eliminated in LDS with the pivots and multipliers of the
-// unblocked elimination (gj_invert).  The panel's row swaps, then its
-// composed elimination T = I + U e_K^T, go to the rest of W in one pass:
-// U = C (I - Lc)^{-1}, where column q of C holds the multipliers of pivot
-// q (c_i = -f_i / p for i /= k, 1/p - 1 at the pivot row) and Lc is the
-// strictly lower part of C's pivot rows.  W is read and written n / B
-// times instead of n times; B <= GJ_BMAX.  lds: gj_lds_bytes<M>(n, B)
-// bytes.  Returns the LAPACK-style info (k + 1 of the first zero pivot, 0
-// if none).
-// ---------------------------------------------------------------------------
-template <class M>
-__device__ int gj_invert_blk(M *W, int n, int nr, M *lds, int B)
-{
-    __shared__ int s_p, s_info, s_piv[GJ_BMAX];
-    __shared__ double s_v[32];
-    __shared__ int s_i[32];
-    M *P = lds, *C = P + (size_t)n * B, *Wk = C + (size_t)n * B, *prow = Wk + B * GJ_CH,
-      *coef = prow + B;
-    const int tid = threadIdx.x, nt = blockDim.x, w2 = 2 * n;
-    if (tid == 0) s_info = 0;
-    for (int t = tid; t < n * nr; t += nt) {
-        const int i = t / nr, j = t - i * nr;
-        W[(size_t)i * w2 + n + j] = i == j ? mk_elem<M>(1.0, 0.0) : mzero<M>();
-    }
-    __syncthreads();
-    for (int k0 = 0; k0 < n; k0 += B) {
-        const int b = min(B, n - k0);
-        for (int t = tid; t < n * B; t += nt) {
-            const int i = t / B, c = t - i * B;
-            P[t] = c < b ? W[(size_t)i * w2 + k0 + c] : mzero<M>();
-            C[t] = mzero<M>();
-        }
-        __syncthreads();
-        // ---- the panel, pivot by pivot, in LDS
-        for (int kk = 0; kk < b; kk++) {
-            const int k = k0 + kk;
-            double bv = -1.0;
-            int bi = n;
-            for (int i = k + tid; i < n; i += nt) {
-                const double v = mabs1(P[(size_t)i * B + kk]);
-                if (v > bv) { bv = v; bi = i; }
-            }
-            for (int o = 32; o > 0; o >>= 1) {
-                const double ov = __shfl_xor(bv, o, 64);
-                const int oi = __shfl_xor(bi, o, 64);
-                if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-            }
-            if ((tid & 63) == 0) { s_v[tid >> 6] = bv; s_i[tid >> 6] = bi; }
-            __syncthreads();
-            if (tid == 0) {
-                double v = s_v[0];
-                int ii = s_i[0];
-                for (int q = 1; q < (nt + 63) / 64; q++)
-                    if (s_v[q] > v || (s_v[q] == v && s_i[q] < ii)) { v = s_v[q]; ii = s_i[q]; }
-                s_p = ii;
-                s_piv[kk] = ii;
-                if (!(v > 0.0) && s_info == 0) s_info = k + 1;
-            }
-            __syncthreads();
-            if (s_info != 0) break;
-            const int p = s_p;
-            if (p != k && tid < B) {
-                const M a = P[(size_t)k * B + tid], c = C[(size_t)k * B + tid];
-                P[(size_t)k * B + tid] = P[(size_t)p * B + tid];
-                C[(size_t)k * B + tid] = C[(size_t)p * B + tid];
-                P[(size_t)p * B + tid] = a;
-                C[(size_t)p * B + tid] = c;
-            }
-            __syncthreads();
-            const M r = mrecip(P[(size_t)k * B + kk]);
-            if (tid < B) prow[tid] = P[(size_t)k * B + tid];
-            for (int i = tid; i < n; i += nt)
-                C[(size_t)i * B + kk] =
-                    i == k ? msub(r, mk_elem<M>(1.0, 0.0)) : mneg(mmm(P[(size_t)i * B + kk], r));
-            __syncthreads();
-            for (int t = tid; t < n * B; t += nt) {
-                const int i = t / B, c = t - i * B;
-                if (c >= kk && c < b) P[t] = madd(P[t], mmm(C[(size_t)i * B + kk], prow[c]));
-            }
-            __syncthreads();
-        }
-        if (s_info != 0) break;
-        // ---- the other columns J = [k0 + b, n) and [n, n + nr): swaps in order
-        const int nl = n - k0 - b, nJ = nl + nr;
-        for (int kk = 0; kk < b; kk++) {
-            const int k = k0 + kk, p = s_piv[kk];
-            if (p != k)
-                for (int jj = tid; jj < nJ; jj += nt) {
-                    const int j = jj < nl ? k0 + b + jj : n + (jj - nl);
-                    const M a = W[(size_t)k * w2 + j];
-                    W[(size_t)k * w2 + j] = W[(size_t)p * w2 + j];
-                    W[(size_t)p * w2 + j] = a;
-                }
-            __syncthreads();
-        }
-        // U = C (I - Lc)^{-1}, in place, last column first
-        for (int kk = b - 1; kk >= 0; kk--) {
-            if (tid < B) coef[tid] = (tid > kk && tid < b) ? C[(size_t)(k0 + tid) * B + kk] : mzero<M>();
-            __syncthreads();
-            for (int i = tid; i < n; i += nt) {
-                M u = C[(size_t)i * B + kk];
-                for (int q = kk + 1; q < b; q++) u = madd(u, mmm(C[(size_t)i * B + q], coef[q]));
-                C[(size_t)i * B + kk] = u;
-            }
-            __syncthreads();
-        }
-        // W[:, J] += U W[K, J], GJ_CH columns at a time
-        for (int j0 = 0; j0 < nJ; j0 += GJ_CH) {
-            const int cw = min(GJ_CH, nJ - j0);
-            for (int t = tid; t < b * cw; t += nt) {
-                const int q = t / cw, jc = t - q * cw, jj = j0 + jc;
-                const int j = jj < nl ? k0 + b + jj : n + (jj - nl);
-                Wk[q * GJ_CH + jc] = W[(size_t)(k0 + q) * w2 + j];
-            }
-            __syncthreads();
-            for (int t = tid; t < n * cw; t += nt) {
-                const int i = t / cw, jc = t - i * cw, jj = j0 + jc;
-                const int j = jj < nl ? k0 + b + jj : n + (jj - nl);
-                M v = W[(size_t)i * w2 + j];
-                for (int q = 0; q < b; q++) v = madd(v, mmm(C[(size_t)i * B + q], Wk[q * GJ_CH + jc]));
-                W[(size_t)i * w2 + j] = v;
-            }
-            __syncthreads();
-        }
-    }
-    __syncthreads();
-    return s_info;
-}
-
 #define PZ_CM(k, n) p.cM[(size_t)(k) * N + (n)]
 #define PZ_CDM(k, n) p.cdM[(size_t)(k) * N + (n)]
 #define PZ_CD2M(k, n) p.cd2M[(size_t)(k) * N + (n)]
 
-// Assembly of the collocation matrices of one (field, m) into the left half
-// of W (row-major, 2n wide), then the scalings of the reference.
+// Max-scaling of the rows of the row-major n x n block W by one workgroup:
+// fac[r] = 1 / max_c |W[r][c]| (the modulus), W[r][c] *= fac[r].  One wave per
+// row, so that the lanes read consecutive addresses.
+template <class M>
+__device__ void coll_scale_rows(M *W, int n, double *fac)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    for (int r = wave; r < n; r += nw) {
+        M *w = W + (size_t)r * n;
+        double mx = 0.0;
+        for (int c = lane; c < n; c += 64) mx = fmax(mx, mabs2(w[c]));
+        const double f = 1.0 / gj_wave_max(mx);
+        for (int c = lane; c < n; c += 64) w[c] = mscale(w[c], f);
+        if (lane == 0) fac[r] = f;
+    }
+    __syncthreads();
+}
+// the same for the columns: fac[c] = 1 / max_r |W[r][c]|; the rows are split
+// over groups of n threads whose maxima meet in red (LDS, blockDim.x values)
+template <class M>
+__device__ void coll_scale_columns(M *W, int n, double *fac, double *red)
+{
+    const int tid = threadIdx.x, nt = blockDim.x, ng = nt / n, g = tid / n, c = tid - g * n;
+    if (g < ng) {
+        double mx = 0.0;
+        for (int r = g; r < n; r += ng) mx = fmax(mx, mabs2(W[(size_t)r * n + c]));
+        red[tid] = mx;
+    }
+    __syncthreads();
+    if (tid < n) {
+        double mx = red[tid];
+        for (int q = 1; q < ng; q++) mx = fmax(mx, red[q * n + tid]);
+        fac[tid] = 1.0 / mx;
+    }
+    __syncthreads();
+    for (int t = tid; t < n * n; t += nt) W[t] = mscale(W[t], fac[t % n]);
+    __syncthreads();
+}
+
+// The columns c < nr of A^{-1} from gj_invert's block and pivot rows to
+// out[c * ldo + k], k < ldo (zero from n on), times frow[c] (scaling of the
+// right-hand side's entry) and fcol[k] (scaling of the unknown), each where
+// given.  16 slots at a time go through tile (LDS, 16 x np values), so that
+// reads and writes are both rows of consecutive addresses.
+template <class M>
+__device__ void coll_store_inverse(const M *W, int n, int nr, char *lds, const double *frow, const double *fcol, M *out,
+                                   int ldo)
+{
+    const GjLayout<M> lay(n);
+    const short *perm = (const short *)(lds + lay.perm);
+    M *tile = (M *)(lds + lay.U);
+    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, np = lay.np;
+    for (int s0 = 0; s0 < n; s0 += 16) {
+        for (int t = tid; t < 16 * n; t += nt) {
+            const int k = t >> 4, s = t & 15;
+            if (s0 + s < n && perm[s0 + s] < nr) tile[s * np + k] = W[(size_t)perm[k] * n + s0 + s];
+        }
+        __syncthreads();
+        for (int s = tid >> 6; s < 16 && s0 + s < n; s += nt >> 6) {
+            const int c = perm[s0 + s];
+            if (c >= nr) continue;
+            for (int k = lane; k < ldo; k += 64) {
+                M v = mzero<M>();
+                if (k < n) v = mscale(tile[s * np + k], (frow ? frow[c] : 1.0) * (fcol ? fcol[k] : 1.0));
+                out[(size_t)c * ldo + k] = v;
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// Assembly of the collocation matrices of one (field, m) into W (row-major,
+// n x n), then the scalings of the reference; red: LDS, blockDim.x doubles.
 //   T / xi: get_tempMat / get_xiMat (update_temp_coll.f90:310-393), rows
 //           preconditioned, fac[r] returned;
 //   psi, m /= 0: get_psiMat (update_psi_coll_smat.f90:674-837), rows then
 //           columns max-scaled, fac[0..2N) rows and fac[2N..4N) columns;
 //   u_phi, m = 0: get_uphiMat (update_psi_coll_smat.f90:919-987).
 template <class M>
-__device__ void coll_assemble(const PzDev &p, const RadView &R, int fld, int m, double hdif, M *W, double *fac)
+__device__ void coll_assemble(const PzDev &p, const RadView &R, int fld, int m, double hdif, M *W, double *fac,
+                              double *red)
 {
     const int N = p.N, nc = p.ncheb, tid = threadIdx.x, nt = blockDim.x;
     const double wimp = p.ss->wimp_lin[0], rn = p.rnorm, dm = (double)m, dm2 = dm * dm;
     const bool psi = fld == 2 && m != 0;
-    const int n = psi ? 2 * N : N, w2 = 2 * n;
+    const int n = psi ? 2 * N : N;
     for (int t = tid; t < n * n; t += nt) {
         const int r = t / n, c = t - r * n;
         M v = mzero<M>();
@@ -311,40 +173,23 @@ __device__ void coll_assemble(const PzDev &p, const RadView &R, int fld, int m, 
             if (cc == 0 || cc == N - 1) { re *= p.boundary_fac; im *= p.boundary_fac; }
             v = mk_elem<M>(re, im);
         }
-        W[(size_t)r * w2 + c] = v;
+        W[t] = v;
     }
     __syncthreads();
-    if (fld < 2 || psi) {
-        // row max-scaling (|.| of the reference: the modulus)
-        for (int r = tid; r < n; r += nt) {
-            double mx = 0.0;
-            for (int c = 0; c < n; c++) mx = fmax(mx, mabs2(W[(size_t)r * w2 + c]));
-            fac[r] = 1.0 / mx;
-            for (int c = 0; c < n; c++) W[(size_t)r * w2 + c] = mscale(W[(size_t)r * w2 + c], fac[r]);
-        }
-        __syncthreads();
-    }
-    if (psi) {
-        for (int c = tid; c < n; c += nt) {
-            double mx = 0.0;
-            for (int r = 0; r < n; r++) mx = fmax(mx, mabs2(W[(size_t)r * w2 + c]));
-            fac[n + c] = 1.0 / mx;
-            for (int r = 0; r < n; r++) W[(size_t)r * w2 + c] = mscale(W[(size_t)r * w2 + c], fac[n + c]);
-        }
-        __syncthreads();
-    }
+    // max-scalings (|.| of the reference: the modulus)
+    if (fld < 2 || psi) coll_scale_rows(W, n, fac);
+    if (psi) coll_scale_columns(W, n, fac + n, red);
 }
 
 // get_omMat / get_psiMat of the influence-matrix method
-// (update_psi_coll_dmat.f90:829-983) into the left half of W (row-major,
-// 2N wide): which = 0 the omega operator (identity minus the implicit
+// (update_psi_coll_dmat.f90:829-983) into W (row-major, N x N): which = 0 the omega operator (identity minus the implicit
 // viscous term), 1 the stream-function operator with beta; zero rows at
 // both walls, boundary_fac on the first and last columns, then the row
 // (fac[0..N)) and column (fac[N..2N)) max-scalings
 __device__ void coll_assemble_dmat(const PzDev &p, const RadView &R, int which, int m, double hdif, double *W,
-                                   double *fac)
+                                   double *fac, double *red)
 {
-    const int N = p.N, nc = p.ncheb, tid = threadIdx.x, nt = blockDim.x, w2 = 2 * N;
+    const int N = p.N, nc = p.ncheb, tid = threadIdx.x, nt = blockDim.x;
     const double wimp = p.ss->wimp_lin[0], rn = p.rnorm, dm2 = (double)m * (double)m;
     for (int t = tid; t < N * N; t += nt) {
         const int r = t / N, c = t - r * N;
@@ -358,31 +203,11 @@ __device__ void coll_assemble_dmat(const PzDev &p, const RadView &R, int which, 
             a = rn * (PZ_CD2M(r, c) + (R.or1(r) + R.beta(r)) * PZ_CDM(r, c) +
                       (R.or1(r) * R.beta(r) + R.dbeta(r) - dm2 * R.or2(r)) * PZ_CM(r, c));
         if (c == 0 || c == N - 1) a *= p.boundary_fac;
-        W[(size_t)r * w2 + c] = a;
+        W[t] = a;
     }
     __syncthreads();
-    for (int r = tid; r < N; r += nt) {
-        double mx = 0.0;
-        for (int c = 0; c < N; c++) mx = fmax(mx, fabs(W[(size_t)r * w2 + c]));
-        fac[r] = 1.0 / mx;
-    }
-    __syncthreads();
-    for (int t = tid; t < N * N; t += nt) {
-        const int r = t / N, c = t - r * N;
-        W[(size_t)r * w2 + c] *= fac[r];
-    }
-    __syncthreads();
-    for (int c = tid; c < N; c += nt) {
-        double mx = 0.0;
-        for (int r = 0; r < N; r++) mx = fmax(mx, fabs(W[(size_t)r * w2 + c]));
-        fac[N + c] = 1.0 / mx;
-    }
-    __syncthreads();
-    for (int t = tid; t < N * N; t += nt) {
-        const int r = t / N, c = t - r * N;
-        W[(size_t)r * w2 + c] *= fac[N + c];
-    }
-    __syncthreads();
+    coll_scale_rows(W, N, fac);
+    coll_scale_columns(W, N, fac + N, red);
 }
 
 // grid (n_m, 3): field 0 = T, 1 = xi, 2 = psi (m /= 0) or u_phi (m = 0);
@@ -391,65 +216,50 @@ __device__ void coll_assemble_dmat(const PzDev &p, const RadView &R, int which, 
 // Forms the inverses, with the reference's scalings folded in, whenever the
 // matrices change (lMat) or when forced; only the first n_r columns of the
 // psi inverse are formed, the ones the m-loop applies.  Dynamic LDS:
-// gj_lds_bytes<cd>(2 n_r, p.gj_b).
+// gj_lds_bytes<cd>(2 n_r).
 __device__ __forceinline__ void build_coll_body(const PzDev &p, int mi, int fld, int force)
 {
     __shared__ double facs[4 * 257];
-    extern __shared__ double2 gj_smem[]; // gj_lds_bytes<cd>(2 n_r, p.gj_b) bytes
+    extern __shared__ double2 gj_smem[]; // gj_lds_bytes<cd>(2 n_r) bytes
     if (!force && p.ss->lMat == 0) return;
     const int N = p.N, m = p.idx2m[mi], tid = threadIdx.x;
     if ((fld == 0 && !p.l_heat) || (fld == 1 && !p.l_chem)) return;
     const RadView R(p.radc, N);
-    char *ws = p.coll_work + (size_t)mi * p.coll_ws;
-    const size_t regT = (size_t)N * 2 * N * sizeof(double);
+    char *ws = p.coll_work + (size_t)mi * p.coll_ws, *lds = (char *)gj_smem;
+    double *red = (double *)gj_smem; // before the inversion
+    const size_t regT = (size_t)N * N * sizeof(double);
     const int ldi = p.ldi;
     if (p.dmat && fld >= 2 && m != 0) {
         // influence-matrix method: field 2 the omega operator, 3 the psi
         // operator; INV = diag(fac_col) A_s^{-1} diag(fac_row), real
         double *W = (double *)(ws + fld * regT);
-        coll_assemble_dmat(p, R, fld - 2, m, p.hdifV[mi], W, facs);
-        const int info = gj_invert_blk<double>(W, N, N, (double *)gj_smem, p.gj_b);
+        coll_assemble_dmat(p, R, fld - 2, m, p.hdifV[mi], W, facs, red);
+        const int info = gj_invert<double>(W, N, N, lds);
         if (tid == 0) p.info[fld * p.nm + mi] = info;
         if (info) return;
-        double *out = (fld == 2 ? p.OmI : p.PsI) + (size_t)mi * N * ldi;
-        for (int t = tid; t < N * ldi; t += blockDim.x) {
-            const int c = t / ldi, r = t - c * ldi;
-            out[(size_t)c * ldi + r] = r < N ? facs[N + r] * W[(size_t)r * 2 * N + N + c] * facs[c] : 0.0;
-        }
+        coll_store_inverse<double>(W, N, N, lds, facs, facs + N, (fld == 2 ? p.OmI : p.PsI) + (size_t)mi * N * ldi, ldi);
         return;
     }
     if (fld == 3) return;
     if (fld < 2 || m == 0) {
-        double *W = (double *)(ws + (fld == 2 ? 2 * regT : fld * regT));
-        coll_assemble<double>(p, R, fld, m, fld == 0 ? p.hdifT[mi] : fld == 1 ? p.hdifXi[mi] : p.hdifV[mi], W, facs);
-        const int info = gj_invert_blk<double>(W, N, N, (double *)gj_smem, p.gj_b);
+        double *W = (double *)(ws + fld * regT);
+        coll_assemble<double>(p, R, fld, m, fld == 0 ? p.hdifT[mi] : fld == 1 ? p.hdifXi[mi] : p.hdifV[mi], W, facs, red);
+        const int info = gj_invert<double>(W, N, N, lds);
         if (tid == 0) p.info[fld * p.nm + mi] = info;
         if (info) return;
         // INV = A_s^{-1} diag(fac) (T, xi); A^{-1} (u_phi); column-major [col][ldi]
         double *out = fld == 0 ? p.T_inv + (size_t)mi * N * ldi : fld == 1 ? p.X_inv + (size_t)mi * N * ldi : p.U_inv;
-        for (int t = tid; t < N * ldi; t += blockDim.x) {
-            const int c = t / ldi, r = t - c * ldi;
-            double v = 0.0;
-            if (r < N) {
-                v = W[(size_t)r * 2 * N + N + c];
-                if (fld < 2) v *= facs[c];
-            }
-            out[(size_t)c * ldi + r] = v;
-        }
+        coll_store_inverse<double>(W, N, N, lds, fld < 2 ? facs : nullptr, nullptr, out, ldi);
     } else {
         cd *W = (cd *)(ws + 2 * regT);
         const int n = 2 * N;
-        coll_assemble<cd>(p, R, fld, m, p.hdifV[mi], W, facs);
-        const int info = gj_invert_blk<cd>(W, n, N, (cd *)gj_smem, p.gj_b);
+        coll_assemble<cd>(p, R, fld, m, p.hdifV[mi], W, facs, red);
+        const int info = gj_invert<cd>(W, n, N, lds);
         if (tid == 0) p.info[fld * p.nm + mi] = info;
         if (info) return;
         // INV = diag(fac_col) A_s^{-1} diag(fac_row); only the first N
         // columns (the omega-equation rows of the right-hand side) are kept
-        cd *out = p.PC_inv + (size_t)mi * N * n;
-        for (int t = tid; t < N * n; t += blockDim.x) {
-            const int c = t / n, r = t - c * n;
-            out[(size_t)c * n + r] = cscale(facs[n + r] * facs[c], W[(size_t)r * 2 * n + n + c]);
-        }
+        coll_store_inverse<cd>(W, n, N, lds, facs, facs + n, p.PC_inv + (size_t)mi * N * n, n);
     }
 }
 
