@@ -637,6 +637,74 @@ static std::vector<double> rhs_band(const pz_handle *h, int K, int nbounds, cons
     return b;
 }
 
+// The m-independent linear maps of the integration m-loop, composed in long
+// double from the bands (T_RHSE1, P_RHSE1, P_RHSE2, P_RHSE3), costf (with and
+// without the modes above n_cheb) and the radial derivative.  All of them
+// follow from the cosine table in O(n_r^2): the derivative of Chebyshev
+// coefficients is a sum over every second higher one, and costf g costf of a
+// radial function g a sum of two cosine coefficients of g.
+static void compose_operators(pz_handle *h, const std::vector<double> &bT, const std::vector<double> &bP0,
+                              const std::vector<double> &bB, const std::vector<double> &bP)
+{
+    const int N = h->N, ldm = (N + 3) & ~3, L = 2 * N - 2, nc = h->ncheb;
+    const ld pi = 3.14159265358979323846264338327950288L, cf = sqrtl(0.5L / (ld)(N - 1));
+    std::vector<ld> ct(L);
+    for (int q = 0; q < L; q++) ct[q] = cosl(pi * (ld)q / (ld)(N - 1));
+    auto wgt = [&](int k) { return k == 0 || k == N - 1 ? 1.0L : 2.0L; };
+    // C[k][j]: costf.  D = costf d/dr costf on coefficients below n_cheb: with
+    // f = cf sum w_k c_k T_k, the coefficients b of df/dx are b_k = b_{k+2} +
+    // 2 (k + 1) a_{k+1} (a = cf w c, b_0 halved), and c' = b / (cf w)
+    std::vector<ld> C((size_t)N * N), D((size_t)N * N, 0.0L);
+    for (int k = 0; k < N; k++)
+        for (int j = 0; j < N; j++) C[(size_t)k * N + j] = cf * wgt(j) * ct[(size_t)j * k % L];
+    for (int j = 0; j < N; j++)
+        for (int k = N - 2; k >= 0; k--) {
+            ld b = k + 2 < N ? D[(size_t)(k + 2) * N + j] : 0.0L;
+            if (k + 1 < nc) b += 2.0L * (k + 1) * wgt(k + 1) * C[(size_t)(k + 1) * N + j];
+            D[(size_t)k * N + j] = b;
+        }
+    for (int k = 0; k < N; k++) {
+        const ld f = (ld)h->drx[0] * (k == 0 ? 0.5L : 1.0L) / wgt(k);
+        for (int j = 0; j < N; j++) D[(size_t)k * N + j] *= f;
+    }
+    // costf g costf, g = -rgrav / r: cf^2 w_l sum_j w_j g_j cos(jk) cos(jl)
+    const pz_config &c = h->c;
+    std::vector<ld> gh(L, 0.0L), G((size_t)N * N);
+    for (int q = 0; q < L; q++)
+        for (int j = 0; j < N; j++) {
+            const double rc = h->r_cmb, rg = c.g0 + c.g1 * h->r[j] / rc + c.g2 * rc * rc * h->or1[j] * h->or1[j];
+            gh[q] -= wgt(j) * (ld)rg * (ld)h->or1[j] * ct[(size_t)j * q % L];
+        }
+    for (int k = 0; k < N; k++)
+        for (int l = 0; l < N; l++) G[(size_t)k * N + l] = 0.5L * cf * cf * wgt(l) * (gh[(k + l) % L] + gh[std::abs(k - l)]);
+    // columns col0 .. of dst: sc times the band times the first n0 rows of B
+    auto band = [&](const std::vector<double> &b, int K, const std::vector<ld> &B, int n0, ld sc, std::vector<double> &dst, int col0) {
+        std::vector<ld> r(N);
+        for (int i = 0; i < N; i++) {
+            std::fill(r.begin(), r.end(), 0.0L);
+            for (int d = -K; d <= K; d++) {
+                const int k = i + d;
+                if (k < 0 || k >= n0) continue;
+                const ld a = sc * (ld)b[(size_t)i * (2 * K + 1) + K + d];
+                if (a == 0.0L) continue;
+                for (int j = 0; j < N; j++) r[j] += a * B[(size_t)k * N + j];
+            }
+            for (int j = 0; j < N; j++) dst[(size_t)(col0 + j) * ldm + i] = (double)r[j];
+        }
+    };
+    std::vector<double> TM((size_t)2 * N * ldm, 0.0), PM(TM), P0((size_t)N * ldm, 0.0), PG(P0);
+    band(bT, 3, C, nc, 1.0L, TM, 0);
+    band(bT, 3, D, nc, -1.0L, TM, N);
+    band(bP, 7, C, nc, 1.0L, PM, 0);
+    band(bP, 7, D, nc, -1.0L, PM, N);
+    band(bP0, 4, C, nc, 1.0L, P0, 0);
+    band(bB, 8, G, N, 1.0L, PG, 0);
+    h->d.T_M = h->upload(TM);
+    h->d.P_M = h->upload(PM);
+    h->d.P_M0 = h->upload(P0);
+    h->d.P_G = h->upload(PG);
+}
+
 static void build_operators(pz_handle *h)
 {
     const int N = h->N, nm = h->nm;
@@ -663,6 +731,8 @@ static void build_operators(pz_handle *h)
         h->d.P_RHSE2 = h->upload(rhs_band(h, 8, 4, s.data()));
         s = rows(7, {&L.I4R3}, {1});
         h->d.P_RHSE3 = h->upload(rhs_band(h, 7, 4, s.data()));
+        compose_operators(h, rhs_band(h, 3, 2, rows(3, {&L.I2R1}, {1}).data()), rhs_band(h, 4, 2, rows(4, {&L.I2R2}, {1}).data()),
+                          rhs_band(h, 8, 4, rows(8, {&L.I4R4}, {1}).data()), rhs_band(h, 7, 4, s.data()));
     }
     std::vector<double> TRHSI((size_t)nm * N * 5, 0.0), PRHSI((size_t)nm * N * 17, 0.0);
     std::vector<double2> PRHSIL((size_t)nm * N * 17, make_double2(0, 0));
@@ -861,7 +931,7 @@ static void allow_full_lds(int lim)
     const void *kernels[] = {(const void *)k_build_lhs, (const void *)k_mphase, (const void *)k_radial_loop,
                              (const void *)k_start, (const void *)k_build_inv, (const void *)k_mcoll,
                              (const void *)k_start_coll, (const void *)k_build_lhs_batch,
-                             (const void *)k_mphase_batch, (const void *)k_radial_loop_batch,
+                             (const void *)k_mphase_batch, (const void *)k_mphase_batch_small, (const void *)k_radial_loop_batch,
                              (const void *)k_build_inv_batch, (const void *)k_mcoll_batch<true>, (const void *)k_mcoll_batch<false>, (const void *)k_fd_build,
                              (const void *)k_fd_mloop, (const void *)k_fd_start, (const void *)k_radial_loop_big,
                              (const void *)k_radial_loop_inplace,
@@ -899,6 +969,7 @@ static void setup(pz_handle *h)
     PzDev &d = h->d;
     d.N = N;
     d.nm = h->nm;
+    d.minc = c.minc;
     d.nphi = h->nphi;
     d.ncheb = c.n_cheb_max;
     d.L = 2 * N - 2;
@@ -1043,8 +1114,6 @@ static void setup(pz_handle *h)
         cosT[q] = (double)cosl(lpi * (ld)q / (ld)(N - 1));
         sinT[q] = (double)sinl(lpi * (ld)q / (ld)(N - 1));
     }
-    d.cosT = h->upload(cosT);
-    d.sinT = h->upload(sinT);
     // bulk factors of get_dr_fft / get_ddr_fft at the interior nodes:
     // 1/(sqrt(1-x^2) nrm), x/((1-x^2)^1.5 nrm), 1/((1-x^2) nrm)
     std::vector<double> drb(3 * N, 0.0);
@@ -1072,7 +1141,15 @@ static void setup(pz_handle *h)
         std::copy(or3.begin(), or3.end(), rc.begin() + (size_t)22 * N);
         std::copy(d2beta.begin(), d2beta.end(), rc.begin() + (size_t)23 * N);
         std::copy(d3beta.begin(), d3beta.end(), rc.begin() + (size_t)24 * N);
-        d.radc = h->upload(rc);
+        // the transform tables and the radial rows form one block
+        // [cos | sin | rows], staged into LDS by one copy (stage_tables)
+        std::vector<double> tab(cosT);
+        tab.insert(tab.end(), sinT.begin(), sinT.end());
+        tab.insert(tab.end(), rc.begin(), rc.end());
+        tab.push_back(0.0); // 16-byte loads of an odd count
+        d.cosT = h->upload(tab);
+        d.sinT = d.cosT + L;
+        d.radc = d.cosT + 2 * L;
         set_radial_pointers(d, d.radc, (size_t)N);
     }
     std::vector<double> tau(6 * N);
@@ -1214,7 +1291,7 @@ static void setup(pz_handle *h)
     // LDS budgets
     h->lds_radial = (5 * (size_t)h->nm + 7 * (size_t)h->nphi) * sizeof(cd) + 16 * sizeof(double);
     h->mthreads = mloop_threads(N);
-    h->lds_mphase = MpLayout(N, h->mthreads).total;
+    h->lds_mphase = MpLayout(N, h->mthreads, true, !d.coll && !d.fd).total;
     h->lds_fd = FdLayout(N).total;
     h->lds_fd_loop = FdLoopLayout(N).total;
     h->lds_start = 15 * (size_t)N * sizeof(cd);
@@ -3047,7 +3124,7 @@ static void launch_class_step(const pz_ensemble *e, const EnsClass &c)
             hipLaunchKernelGGL(c.rad_lds ? k_mcoll_batch<true> : k_mcoll_batch<false>, dim3(c.nb_m), dim3(c.mthreads),
                                c.lds_m, c.stream, PzBatch{runs, c.map_m, (int)c.members.size()}, stage, exp_calc);
         else
-            hipLaunchKernelGGL(k_mphase_batch, dim3(c.nb_m), dim3(c.mthreads), c.lds_m, c.stream,
+            hipLaunchKernelGGL(c.n <= 65 ? k_mphase_batch_small : k_mphase_batch, dim3(c.nb_m), dim3(c.mthreads), c.lds_m, c.stream,
                                PzBatch{runs, c.map_m, (int)c.members.size()}, stage, exp_calc);
     }
 }

@@ -400,20 +400,20 @@ __device__ __forceinline__ void coll_uphi0_impl(const PzDev &p, const RadView &R
         VecSet<cd> dout(cA);
         dct_fft(p, din, dout, 1, 0, cosT, sinT, fbuf);
     }
-    __syncthreads();
+    lds_barrier();
     double *f = dt3, *df = dt3 + N, *ddf = dt3 + 2 * N;
     for (int k = tid; k < N; k += blockDim.x) f[k] = cA[k].x;
-    __syncthreads();
+    lds_barrier();
     if (tid == 0) ddcheb_real(p, f, df, ddf);
-    __syncthreads();
+    lds_barrier();
     for (int k = tid; k < N; k += blockDim.x) { cA[k] = mk(df[k], 0.0); cB[k] = mk(ddf[k], 0.0); }
-    __syncthreads();
+    lds_barrier();
     {
         const VecSet<const cd> din(cA, cB);
         VecSet<cd> dout(cA, cB);
         dct_fft(p, din, dout, 2, 0, cosT, sinT, fbuf);
     }
-    __syncthreads();
+    lds_barrier();
     for (int k = tid; k < N; k += blockDim.x) {
         const double a = R.drx(k), b = R.ddrx(k);
         const double d1 = a * cA[k].x, d2 = b * cA[k].x + a * a * cB[k].x, u = u0[k].x;
@@ -491,7 +491,7 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
     const double wcur = imex_weight(p, ss, istage);
     // the groups above wrote vectors that other threads read next, with or
     // without the explicit part
-    __syncthreads();
+    lds_barrier();
 
     // ---------------- explicit part --------------------------------------
     if (exp_calc) {
@@ -503,7 +503,7 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
             din.push(aP); dout.push(cP);
             dct_fft(p, din, dout, din.n, 0, cosT, sinT, fbuf);
         }
-        __syncthreads();
+        lds_barrier();
         {
             VecSet<const cd> c3;
             VecSet<cd> d3;
@@ -512,7 +512,7 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
             c3.push(cP); d3.push(aP);
             dr_fft(p, R, c3, d3, VecSet<cd>(), c3.n, cosT, sinT, fbuf);
         }
-        __syncthreads();
+        lds_barrier();
         for (int k = tid; k < N; k += blockDim.x) {
             const double o1 = R.or1(k);
             if (hT) {
@@ -559,7 +559,7 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
             aX[k] = r;
         }
     }
-    __syncthreads();
+    lds_barrier();
     if (hT && hX) {
         const VecSet<const double> inv(p.T_inv + off * ldi, p.X_inv + off * ldi);
         const VecSet<cd> xs(aT, aX);
@@ -570,7 +570,7 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
         block_matvec<double, 1>(N, ldi, inv, xs, xs, red);
     }
     for (int k = nc + tid; k < N; k += blockDim.x) { aT[k] = mk(0, 0); aX[k] = mk(0, 0); }
-    __syncthreads();
+    lds_barrier();
     const int inext = (istage == p.nstages) ? 1 : istage + 1;
     // implicit terms for the next stage; also before a CNAB2 start-up step
     // of a multistep scheme, which recomputes them (step_time.f90:417-503)
@@ -579,11 +579,11 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
         // get_ddr (coefficients in) and costf: derivatives and grid values
         if (hT) {
             dr_fft(p, R, VecSet<const cd>(aT), VecSet<cd>(cT), VecSet<cd>(bv), 1, cosT, sinT, fbuf, Tv);
-            __syncthreads();
+            lds_barrier();
         }
         if (hX) {
             dr_fft(p, R, VecSet<const cd>(aX), VecSet<cd>(cX), VecSet<cd>(b2), 1, cosT, sinT, fbuf, Xv);
-            __syncthreads();
+            lds_barrier();
         }
     } else {
         VecSet<const cd> din;
@@ -591,11 +591,11 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
         if (hT) { din.push(aT); dout.push(Tv); }
         if (hX) { din.push(aX); dout.push(Xv); }
         if (din.n) dct_fft(p, din, dout, din.n, 0, cosT, sinT, fbuf);
-        __syncthreads();
+        lds_barrier();
     }
     if (hT) rotate_row(p, p.T_old, p.T_impl, p.T_expl, off);
     if (hX) rotate_row(p, p.X_old, p.X_impl, p.X_expl, off);
-    __syncthreads();
+    lds_barrier();
     for (int k = tid; k < N; k += blockDim.x) {
         const double o1 = R.or1(k), o2 = R.or2(k);
         if (hT) {
@@ -616,7 +616,7 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
             }
         }
     }
-    __syncthreads();
+    lds_barrier();
 
     // ---------------- psi / omega / u_phi ---------------------------------
     const double wl = ss->wimp_lin[0];
@@ -626,24 +626,24 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
             const cd r = cadd(cadd(PP[k], cscale(wcur, eP[k])), QP[k]);
             wv[k] = (k == 0 || k == N - 1) ? mk(0, 0) : mk(r.x, 0.0);
         }
-        __syncthreads();
+        lds_barrier();
         block_matvec<double, 1>(N, ldi, VecSet<const double>(p.U_inv), VecSet<cd>(wv), VecSet<cd>(wv), red);
         for (int k = nc + tid; k < N; k += blockDim.x) wv[k] = mk(0, 0);
-        __syncthreads();
+        lds_barrier();
         // om0 = get_dr(uphi0, l_dct = .false.) (dcheb recursion), uphi0 -> grid
         double *f = (double *)b2, *df = f + N;
         for (int k = tid; k < N; k += blockDim.x) f[k] = wv[k].x;
-        __syncthreads();
+        lds_barrier();
         if (tid == 0) dcheb_real(p, f, df);
-        __syncthreads();
+        lds_barrier();
         for (int k = tid; k < N; k += blockDim.x) { cP[k] = mk(df[k], 0.0); eP[k] = mk(f[k], 0.0); }
-        __syncthreads();
+        lds_barrier();
         {
             const VecSet<const cd> din(cP, eP);
             VecSet<cd> dout(omv, upv);
             dct_fft(p, din, dout, 2, 0, cosT, sinT, fbuf);
         }
-        __syncthreads();
+        lds_barrier();
         for (int k = tid; k < N; k += blockDim.x) {
             const double u0 = upv[k].x, om0 = R.drx(k) * omv[k].x;
             const cd om = mk(om0 + R.or1(k) * u0, 0.0);
@@ -655,12 +655,12 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
             p.psi[off + k] = mk(0, 0);
         }
         rotate_row(p, p.P_old, p.P_impl, p.P_expl, off);
-        __syncthreads();
+        lds_barrier();
         if (inext == 1)
             for (int k = tid; k < N; k += blockDim.x) p.P_old[off + k] = upv[k];
         if (lcalc)
             coll_uphi0_impl(p, R, upv, cP, eP, (double *)bv, cosT, sinT, fbuf, wv, p.hdifV[mi]);
-        __syncthreads();
+        lds_barrier();
         if (lcalc)
             for (int k = tid; k < N; k += blockDim.x) p.P_impl[(inext - 1) * F + off + k] = wv[k];
         return;
@@ -673,21 +673,21 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
         }
         aP[k] = (k == 0 || k == N - 1) ? mk(0, 0) : r;
     }
-    __syncthreads();
+    lds_barrier();
     if (p.dmat) {
         // update_om_coll_dmat (update_psi_coll_dmat.f90:244-453): omega_1
         // from its own equation (omega = 0 at the walls) ...
         block_matvec<double, 1>(N, ldi, VecSet<const double>(p.OmI + off * ldi), VecSet<cd>(aP), VecSet<cd>(aP), red);
         for (int k = nc + tid; k < N; k += blockDim.x) aP[k] = mk(0, 0);
-        __syncthreads();
+        lds_barrier();
         dct_fft(p, VecSet<const cd>(aP), VecSet<cd>(eP), 1, 0, cosT, sinT, fbuf);
-        __syncthreads();
+        lds_barrier();
         // ... psi_1 from L_psi psi = -omega_1 (psi = 0 at the walls) ...
         for (int k = tid; k < N; k += blockDim.x) cP[k] = (k == 0 || k == N - 1) ? mk(0, 0) : mk(-eP[k].x, -eP[k].y);
-        __syncthreads();
+        lds_barrier();
         block_matvec<double, 1>(N, ldi, VecSet<const double>(p.PsI + off * ldi), VecSet<cd>(cP), VecSet<cd>(cP), red);
         for (int k = nc + tid; k < N; k += blockDim.x) cP[k] = mk(0, 0);
-        __syncthreads();
+        lds_barrier();
         // ... and the multiples of the homogeneous pairs that meet the
         // velocity conditions (solve_influence_matrix, :1256-1300)
         double tx = 0.0, ty = 0.0, bx = 0.0, by = 0.0;
@@ -709,21 +709,21 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
             aP[k] = cadd(cadd(aP[k], cscale(hom[k], c1)), cscale(hom[N + k], c2));
             cP[k] = cadd(cadd(cP[k], cscale(hom[2 * N + k], c1)), cscale(hom[3 * N + k], c2));
         }
-        __syncthreads();
+        lds_barrier();
     } else {
         // [omega; psi] coefficients (2N values in aP, cP)
         block_matvec_rc<cd, 1>(2 * N, N, 2 * N, VecSet<const cd>(p.PC_inv + off * 2 * N), VecSet<cd>(aP),
                                VecSet<cd>(aP), red);
         for (int k = nc + tid; k < N; k += blockDim.x) { aP[k] = mk(0, 0); cP[k] = mk(0, 0); }
-        __syncthreads();
+        lds_barrier();
     }
     // d psi / dr and psi on the grid
     dr_fft(p, R, VecSet<const cd>(cP), VecSet<cd>(eP), VecSet<cd>(), 1, cosT, sinT, fbuf, psiv);
-    __syncthreads();
+    lds_barrier();
     // omega on the grid, with its derivatives for the implicit term
     if (lcalc) dr_fft(p, R, VecSet<const cd>(aP), VecSet<cd>(bv), VecSet<cd>(b2), 1, cosT, sinT, fbuf, omv);
     else dct_fft(p, VecSet<const cd>(aP), VecSet<cd>(omv), 1, 0, cosT, sinT, fbuf);
-    __syncthreads();
+    lds_barrier();
     for (int k = tid; k < N; k += blockDim.x) {
         const cd ps = psiv[k];
         const cd us = cmul(mk(0.0, dm * R.or1(k)), ps);
@@ -736,7 +736,7 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
         p.om[off + k] = omv[k];
     }
     rotate_row(p, p.P_old, p.P_impl, p.P_expl, off);
-    __syncthreads();
+    lds_barrier();
     for (int k = tid; k < N; k += blockDim.x) {
         if (inext == 1) p.P_old[off + k] = omv[k];
         if (lcalc) {

@@ -80,6 +80,19 @@ __device__ __forceinline__ void lds_store(cd *q, int i, cd v)
     d[2 * i + 1] = v.y;
 }
 
+// Barrier of the workgroup that orders LDS accesses only.  __syncthreads also
+// waits for every outstanding global load and store of the wave, which keeps
+// a phase's result stores (one to two microseconds) and loads issued ahead of
+// their use on the chain; between phases that exchange values through LDS
+// alone nothing needs them.  Where another thread reads global memory written
+// before the barrier, __syncthreads stays.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Loads through a generic pointer known to address global memory, retyped
 // so that they compile to global_load (which counts only against vmcnt)
 // instead of flat loads, whose waits also stall on pending LDS accesses.
@@ -248,7 +261,7 @@ __device__ cd *fft_stockham(cd *a, cd *b, int n, int ntr, int dir, const int *ra
                 }
                 b[tr * n + (j / Ns) * Ns * R + jm + k * Ns] = acc;
             }
-            __syncthreads();
+            lds_barrier();
             cd *t = a;
             a = b;
             b = t;
@@ -281,7 +294,7 @@ __device__ cd *fft_stockham(cd *a, cd *b, int n, int ntr, int dir, const int *ra
                 y[idxD] = v[0]; y[idxD + Ns] = v[1]; y[idxD + 2 * Ns] = v[2];
             }
         }
-        __syncthreads();
+        lds_barrier();
         cd *t = a;
         a = b;
         b = t;
@@ -313,13 +326,13 @@ __device__ __forceinline__ void inplace_bfly(cd *a, int n, int ntr, int Ns, int 
             d[it] = tr * n + (j / Ns) * Ns * R + jm;
         }
     }
-    __syncthreads();
+    lds_barrier();
 #pragma unroll
     for (int it = 0; it < IT; it++)
         if (d[it] >= 0)
 #pragma unroll
             for (int r = 0; r < R; r++) a[d[it] + r * Ns] = y[it][r];
-    __syncthreads();
+    lds_barrier();
 }
 // one Horner step a z + v
 __device__ __forceinline__ cd hstep(cd a, cd z, cd v)
@@ -359,13 +372,13 @@ __device__ __forceinline__ void inplace_prime(cd *a, int n, int ntr, int Ns, int
             cnt[it] = min(G, R - k0);
         }
     }
-    __syncthreads();
+    lds_barrier();
 #pragma unroll
     for (int it = 0; it < IT; it++)
 #pragma unroll
         for (int c = 0; c < G; c++)
             if (c < cnt[it]) a[d[it] + c * Ns] = y[it][c];
-    __syncthreads();
+    lds_barrier();
 }
 // The first stage of a plan (no twiddles) with an odd prime R, 5 <= R <=
 // 31: the R-point DFT by conjugate pairs.  With s_j = x_j + x_{R-j}, d_j =
@@ -388,7 +401,7 @@ __device__ __forceinline__ void inplace_prime_first(cd *a, int n, int ntr, int R
         const int j = e / PZ_SYM_ROW + 1, k = e - (j - 1) * PZ_SYM_ROW + 1;
         om[e] = tw(((j * k) % R) * nb);
     }
-    __syncthreads();
+    lds_barrier();
     cd y[2 * P + 1];
     int base = 0, kl = 1, cnt = 0;
     const int t = threadIdx.x;
@@ -426,7 +439,7 @@ __device__ __forceinline__ void inplace_prime_first(cd *a, int n, int ntr, int R
         cnt = min(P, h + 1 - kl);
         if (g == 0) cnt = -1 - cnt; // X_0 as well
     }
-    __syncthreads();
+    lds_barrier();
     const int np = cnt < 0 ? -1 - cnt : cnt;
 #pragma unroll
     for (int c = 0; c < P; c++)
@@ -435,7 +448,7 @@ __device__ __forceinline__ void inplace_prime_first(cd *a, int n, int ntr, int R
             a[base + R - kl - c] = y[2 * c + 1];
         }
     if (cnt < 0) a[base] = y[2 * P];
-    __syncthreads();
+    lds_barrier();
 }
 // om: LDS for PZ_FFT_OM_MAX entries, used when the plan starts with an odd
 // prime 5 <= R <= 31 (one item per thread there: fft_inplace_fits)
@@ -643,12 +656,12 @@ __device__ double block_reduce(double v, double *scratch, int op /*0 sum, 1 max*
         double u = __shfl_xor(v, o, 64);
         v = op == 0 ? v + u : fmax(v, u);
     }
-    __syncthreads();
+    lds_barrier();
     if (lane == 0) scratch[w] = v;
-    __syncthreads();
+    lds_barrier();
     double r = scratch[0];
     for (int i = 1; i < nw; i++) r = op == 0 ? r + scratch[i] : fmax(r, scratch[i]);
-    __syncthreads();
+    lds_barrier();
     return r;
 }
 
@@ -677,7 +690,7 @@ __device__ __forceinline__ void radial_loop_body(const PzDev &p, int nr, int is,
         spec[3 * nm + i] = p.l_heat ? p.temp[q] : mk(0, 0);
         spec[4 * nm + i] = p.l_chem ? p.xi[q] : mk(0, 0);
     }
-    __syncthreads();
+    lds_barrier();
     // Reynolds-stress m-sum (radial_loop.f90:267-278)
     double part = 0.0;
     for (int i = threadIdx.x; i < nm; i += blockDim.x) {
@@ -704,14 +717,14 @@ __device__ __forceinline__ void radial_loop_body(const PzDev &p, int nr, int is,
     if (Pw) {
         fft_wave_phi(Pw, nin, packed, [=](int tr, int k, cd v) { bufb[tr * n + k] = v; },
                      [=](int k) { const cd w = twl[k]; return mk(w.x, -w.y); });
-        __syncthreads();
+        lds_barrier();
         g = bufb;
     } else {
         for (int t = threadIdx.x; t < nin * n; t += blockDim.x) {
             const int tr = t / n;
             bufa[t] = packed(tr, t - tr * n);
         }
-        __syncthreads();
+        lds_barrier();
         g = fft_stockham(bufa, bufb, n, nin, +1, p.radices, p.nrad,
                          [&](int k) { const cd w = twl[k]; return mk(w.x, -w.y); });
     }
@@ -750,13 +763,13 @@ __device__ __forceinline__ void radial_loop_body(const PzDev &p, int nr, int is,
             o[(p.l_heat ? 2 : 1) * n + j] = mk(up * X, rr * us * X);
         }
     }
-    __syncthreads();
+    lds_barrier();
     cd *other = (o == bufa) ? bufb : bufa;
     cd *Z;
     if (Pw) {
         fft_wave_phi(Pw, nout, [=](int tr, int i) { return o[tr * n + i]; },
                      [=](int tr, int k, cd v) { other[tr * n + k] = v; }, [=](int k) { return twl[k]; });
-        __syncthreads();
+        lds_barrier();
         Z = other;
     } else {
         Z = fft_stockham(o, other, n, nout, -1, p.radices, p.nrad, [&](int k) { return twl[k]; });
@@ -837,21 +850,21 @@ __device__ __forceinline__ void radial_loop_big_body(const PzDev &p, int nr, int
         }
         (tr == 0 ? s0 : (tr == 1 ? s1 : s2))[k] = z;
     }
-    __syncthreads();
+    lds_barrier();
     // one complex FFT at a time; the result lands in the column or in the
     // scratch, whose roles are then exchanged
     {
         cd *g = fft_stockham(s0, sc, n, 1, +1, p.radices, p.nrad, bwd);
         if (g != s0) { sc = s0; s0 = g; }
-        __syncthreads();
+        lds_barrier();
         g = fft_stockham(s1, sc, n, 1, +1, p.radices, p.nrad, bwd);
         if (g != s1) { sc = s1; s1 = g; }
         if (p.l_chem) {
-            __syncthreads();
+            lds_barrier();
             g = fft_stockham(s2, sc, n, 1, +1, p.radices, p.nrad, bwd);
             if (g != s2) { sc = s2; s2 = g; }
         }
-        __syncthreads();
+        lds_barrier();
     }
     if (courant) {
         double vr = 0.0, vh = 0.0;
@@ -883,21 +896,21 @@ __device__ __forceinline__ void radial_loop_big_body(const PzDev &p, int nr, int
         s1[j] = mk(up * T, rr * us * T);
         if (p.l_chem) s2[j] = mk(up * X, rr * us * X);
     }
-    __syncthreads();
+    lds_barrier();
     {
         cd *g = fft_stockham(s0, sc, n, 1, -1, p.radices, p.nrad, fwd);
         if (g != s0) { sc = s0; s0 = g; }
         if (p.l_heat) {
-            __syncthreads();
+            lds_barrier();
             g = fft_stockham(s1, sc, n, 1, -1, p.radices, p.nrad, fwd);
             if (g != s1) { sc = s1; s1 = g; }
         }
         if (p.l_chem) {
-            __syncthreads();
+            lds_barrier();
             g = fft_stockham(s2, sc, n, 1, -1, p.radices, p.nrad, fwd);
             if (g != s2) { sc = s2; s2 = g; }
         }
-        __syncthreads();
+        lds_barrier();
     }
     // unpack, normalise and post-scale (radial_loop.f90:350-386)
     const double or1 = p.or1[nr];
@@ -981,7 +994,7 @@ __device__ __forceinline__ void radial_loop_inplace_body(const PzDev &p, int nr,
     }
     for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
     if ((threadIdx.x & 63) == 0) msr[threadIdx.x >> 6] = part;
-    __syncthreads();
+    lds_barrier();
     fft_inplace(s0, n, 2, +1, p.radices, p.nrad, bwd, om);
     if (courant) {
         double vr = 0.0, vh = 0.0;
@@ -1011,7 +1024,7 @@ __device__ __forceinline__ void radial_loop_inplace_body(const PzDev &p, int nr,
         s0[j] = mk(up * om, rr * us * om);
         s1[j] = mk(up * T, rr * us * T);
     }
-    __syncthreads();
+    lds_barrier();
     fft_inplace(s0, n, p.l_heat ? 2 : 1, -1, p.radices, p.nrad, fwd, om);
     // unpack, normalise and post-scale (radial_loop.f90:350-386)
     const double or1 = p.or1[nr];
@@ -1717,7 +1730,7 @@ __device__ __forceinline__ void dct_fft(const PzDev &p, VecSet<const cd> in, Vec
         const int f = t / L, j = t - f * L;
         A[t] = lds_load(in[f], j < N ? j : L - j);
     }
-    __syncthreads();
+    lds_barrier();
     const cd *Z = fft_cheb(p, A, B, nf, -1, cosT, sinT);
     const double cf = p.cheb_fac;
     for (int t = threadIdx.x; t < nf * N; t += blockDim.x) {
@@ -1810,7 +1823,7 @@ __device__ __forceinline__ void dr_fft(const PzDev &p, const RadView &R, VecSet<
             }
         }
     }
-    __syncthreads();
+    lds_barrier();
     const cd *Z = P ? A : fft_cheb(p, A, B, ntr, -1, cosT, sinT);
     for (int t = threadIdx.x; t < nf * N; t += blockDim.x) {
         const int f = t / N, j = t - f * N;
@@ -1863,10 +1876,10 @@ __device__ __forceinline__ void bandmv(const PzDev &p, const double *band, const
                 }
             }
         }
-        sx += __shfl_xor(sx, 1, G);
-        sy += __shfl_xor(sy, 1, G);
-        sx += __shfl_xor(sx, 2, G);
-        sy += __shfl_xor(sy, 2, G);
+        sx += xor_lane_d<1>(sx);
+        sy += xor_lane_d<1>(sy);
+        sx += xor_lane_d<2>(sx);
+        sy += xor_lane_d<2>(sy);
         if (sub == 0) y[i] = mk(sx, sy);
     }
 }
@@ -1890,10 +1903,10 @@ __device__ __forceinline__ void bandmv_c(const PzDev &p, const cd *band, const c
                 if (d < W && jj >= 0 && jj < N) s = cadd(s, cmul(b[u], lds_load(x, jj)));
             }
         }
-        s.x += __shfl_xor(s.x, 1, G);
-        s.y += __shfl_xor(s.y, 1, G);
-        s.x += __shfl_xor(s.x, 2, G);
-        s.y += __shfl_xor(s.y, 2, G);
+        s.x += xor_lane_d<1>(s.x);
+        s.y += xor_lane_d<1>(s.y);
+        s.x += xor_lane_d<2>(s.x);
+        s.y += xor_lane_d<2>(s.y);
         if (sub == 0) y[i] = s;
     }
 }
@@ -2256,6 +2269,34 @@ __device__ __forceinline__ void lds_copy(void *dst, const void *src, size_t byte
     }
 }
 
+// The block [cos | sin | radial rows] of n doubles from global memory to LDS
+// (both 16-byte aligned, n rounded up to even): the first loads of each thread
+// are issued by load(), together with a kernel's other inputs, and stored by
+// store().
+struct TableStage {
+    static constexpr int U = 6; // covers n_r 197 with 512 threads, 65 with 256
+    double2 v[U];
+    __device__ __forceinline__ void load(const double *src, int n)
+    {
+        const int n2 = (n + 1) >> 1;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (u * (int)blockDim.x >= n2) break;
+            v[u] = gld2(src + 2 * min((int)threadIdx.x + u * (int)blockDim.x, n2 - 1));
+        }
+    }
+    __device__ __forceinline__ void store(const double *src, double *dst, int n) const
+    {
+        const int n2 = (n + 1) >> 1;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = threadIdx.x + u * blockDim.x;
+            if (i < n2) lds_store((cd *)dst, i, v[u]);
+        }
+        for (int i = threadIdx.x + U * blockDim.x; i < n2; i += blockDim.x) lds_store((cd *)dst, i, gld2(src + 2 * i));
+    }
+};
+
 // ---------------------------------------------------------------------------
 // Dense solve by explicit inverse: y_i = sum_j INV[j][i] x_j (i < nrow,
 // j < ncol) for NMAT matrices at once (column-major, leading dimension
@@ -2324,7 +2365,7 @@ __device__ __forceinline__ void block_matvec_rc(int nrow, int ncol, int ldi, Vec
 #pragma unroll
                 for (int r = 0; r < RPT; r++) lds_store(red, (size_t)a * RS + (cg - 1) * R * RPT + ru * RPT + r, acc[a][r]);
     }
-    __syncthreads();
+    lds_barrier();
     if (cg == 0) {
 #pragma unroll
         for (int a = 0; a < NMAT; a++)
@@ -2336,7 +2377,7 @@ __device__ __forceinline__ void block_matvec_rc(int nrow, int ncol, int ldi, Vec
                 if (row < nrow) lds_store(y[a], row, s);
             }
     }
-    __syncthreads();
+    lds_barrier();
 }
 // square n x n form
 template <class E, int NMAT>
@@ -2344,6 +2385,102 @@ __device__ __forceinline__ void block_matvec(int N, int ldi, VecSet<const E> inv
                                              cd *red)
 {
     block_matvec_rc<E, NMAT>(N, N, ldi, inv, x, y, red);
+}
+
+// The first PF column loads of a thread of block_matvec_rc, issued long before
+// the product: the same split of rows and columns, the same sums.
+template <class E, int NMAT, int PF>
+struct MatAhead {
+    double2 v[NMAT][PF];
+    static constexpr int RPT = sizeof(E) == 8 ? 2 : 1;
+    __device__ __forceinline__ void load(int nrow, int ncol, int ldi, VecSet<const E> inv)
+    {
+        const int R = (nrow + RPT - 1) / RPT, CG = min((int)blockDim.x / R, ncol);
+        const int cg = threadIdx.x / R, ru = threadIdx.x - cg * R;
+#pragma unroll
+        for (int u = 0; u < PF; u++) {
+            const int jj = cg + u * CG;
+            const bool ok = cg < CG && jj < ncol;
+#pragma unroll
+            for (int a = 0; a < NMAT; a++)
+                v[a][u] = ok ? gld2((const double *)(inv[a] + (size_t)jj * ldi + (size_t)ru * RPT)) : mk(0.0, 0.0);
+        }
+    }
+    // y = INV x (x and y may alias; every thread of the block calls it): all
+    // column groups' partial sums go to red (ahead_scratch values), and one
+    // thread per row adds them up in the order of the groups and hands them to
+    // out(row, sums); mid() comes last, at once on the waves without rows
+    template <class MID, class OUT>
+    __device__ __forceinline__ void apply(int nrow, int ncol, int ldi, VecSet<const E> inv, VecSet<cd> x, cd *red, MID mid,
+                                          OUT out) const
+    {
+        constexpr int U = 16 / NMAT;
+        const int R = (nrow + RPT - 1) / RPT, CG = min((int)blockDim.x / R, ncol);
+        const int cg = threadIdx.x / R, ru = threadIdx.x - cg * R;
+        const int RW = R * RPT, RS = CG * RW;
+        cd acc[NMAT][RPT];
+#pragma unroll
+        for (int a = 0; a < NMAT; a++)
+#pragma unroll
+            for (int r = 0; r < RPT; r++) acc[a][r] = mk(0.0, 0.0);
+        auto add = [&](int a, double2 w, int jj) __attribute__((always_inline)) {
+            const cd xj = lds_load(x[a], jj);
+            if constexpr (RPT == 2) {
+                acc[a][0].x = fma(w.x, xj.x, acc[a][0].x);
+                acc[a][0].y = fma(w.x, xj.y, acc[a][0].y);
+                acc[a][1].x = fma(w.y, xj.x, acc[a][1].x);
+                acc[a][1].y = fma(w.y, xj.y, acc[a][1].y);
+            } else {
+                acc[a][0] = cadd(acc[a][0], cmul(w, xj));
+            }
+        };
+        if (cg < CG) {
+            const int nj = (ncol - cg + CG - 1) / CG;
+#pragma unroll
+            for (int u = 0; u < PF; u++) {
+                const int jj = min(cg + u * CG, ncol - 1); // columns past the end were loaded as zeros
+#pragma unroll
+                for (int a = 0; a < NMAT; a++) add(a, v[a][u], jj);
+            }
+            for (int jb = PF; jb < nj; jb += U) {
+                double2 w[NMAT][U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int jj = cg + (jb + u) * CG;
+#pragma unroll
+                    for (int a = 0; a < NMAT; a++)
+                        w[a][u] = jb + u < nj ? gld2((const double *)(inv[a] + (size_t)jj * ldi + (size_t)ru * RPT)) : mk(0.0, 0.0);
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const int jj = min(cg + (jb + u) * CG, ncol - 1);
+#pragma unroll
+                    for (int a = 0; a < NMAT; a++) add(a, w[a][u], jj);
+                }
+            }
+#pragma unroll
+            for (int a = 0; a < NMAT; a++)
+#pragma unroll
+                for (int r = 0; r < RPT; r++) lds_store(red, a * RS + cg * RW + ru * RPT + r, acc[a][r]);
+        }
+        lds_barrier();
+        for (int k = threadIdx.x; k < nrow; k += blockDim.x) {
+            cd s[NMAT];
+#pragma unroll
+            for (int a = 0; a < NMAT; a++) {
+                s[a] = lds_load(red, a * RS + k);
+                for (int c = 1; c < CG; c++) s[a] = cadd(s[a], lds_load(red, a * RS + c * RW + k));
+            }
+            out(k, s);
+        }
+        mid();
+    }
+};
+// complex values of red for that product
+__host__ __device__ inline size_t ahead_scratch(int nrow, int ncol, int threads, int rpt, int nmat)
+{
+    const int R = (nrow + rpt - 1) / rpt, CG = threads / R < ncol ? threads / R : ncol;
+    return (size_t)nmat * CG * R * rpt;
 }
 
 // LDS layout of k_build_inv: one field's bordered factors (sized for the

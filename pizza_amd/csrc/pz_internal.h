@@ -48,6 +48,7 @@ struct PzBatch {
 // Everything a kernel needs: sizes, constants and device pointers.
 struct PzDev {
     int N, nm, nphi, ncheb, L; // L = 2N-2 (Chebyshev even extension)
+    int minc;                  // mode i has m = i minc (idx2m)
     int family, nstages, nexp, nimp, nold;
     int scheme, bridge; // enum pz_time_scheme; 1: multistep start-up steps use CNAB2
     int l_heat, l_chem, l_coriolis_imp, l_buo_imp, l_ek_pump;
@@ -98,6 +99,13 @@ struct PzDev {
     // (entry K+d is column i+d), already multiplied by rnorm
     const double *T_RHSE1, *T_RHSE2;           // K = 3, 4
     const double *P_RHSE1, *P_RHSE2, *P_RHSE3; // K = 4, 8, 7
+    // m-independent maps of the integration m-loop composed from the
+    // transforms, the radial derivative and those bands, column-major
+    // [col][n_r rounded up to 4]: [band costf | -band costf d/dr] of the explicit assembly of
+    // T and xi (T_M) and of psi (P_M; m = 0: P_M0, band costf alone), 2 n_r
+    // (n_r) columns, and the implicit buoyancy's band costf (-rgrav / r)
+    // costf (P_G) on Chebyshev coefficients
+    const double *T_M, *P_M, *P_M0, *P_G;
     // per-m RHS bands
     const double *T_RHSI; // [nm][n_r][5]  K = 2
     const double *P_RHSI; // [nm][n_r][17] K = 8 (m = 0 uses the central 9)

@@ -1,0 +1,51 @@
+"""The integration method's m-loop at the sizes and options where its shared
+products, their column groups and its transforms take another form: the
+smallest n_r, both thread counts (n_r 65 and 66), register FFTs (33, 97) and
+Stockham FFTs, both limits of the column groups (160 and 161), the largest
+n_r; fewer Chebyshev modes than radii; T alone, xi alone and both; implicit
+and explicit buoyancy; every slot of SBDF4 and the stage sums of ARS443.
+Two steps against the oracle, each field within ten times what one rounding
+of dt moves the oracle's own result (its conditioning), and at least 1e-11."""
+import pytest
+
+from helpers import rel
+from test_gpu_parity import _fields, _floor, _pair
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # n_r, n_cheb, scheme, ra, raxi, buoyancy, pumping
+    (8, 8, "CNAB2", 1e5, 1e5, "IMP", True),
+    (33, 33, "SBDF4", 1e6, 0.0, "IMP", False),
+    (33, 27, "ARS443", 0.0, 1e6, "IMP", True),
+    (48, 48, "CNLF", 1e6, 1e6, "EXP", True),
+    (65, 52, "SBDF2", 1e6, 1e6, "IMP", True),
+    (66, 66, "BPR353", 1e6, 1e6, "IMP", False),
+    (97, 80, "BPR353", 1e6, 0.0, "EXP", True),
+    (98, 98, "MODCNAB", 0.0, 1e6, "EXP", False),
+    (129, 129, "ARS443", 1e6, 1e6, "IMP", True),
+    (160, 160, "CNAB2", 1e6, 1e6, "IMP", False),
+    (161, 161, "CNAB2", 1e6, 1e6, "IMP", True),
+    (198, 198, "BPR353", 1e6, 1e6, "IMP", True),
+]
+
+
+@pytest.mark.parametrize("n_r,n_cheb,scheme,ra,raxi,buo,pump", CASES)
+def test_integ_mloop_sizes(n_r, n_cheb, scheme, ra, raxi, buo, pump):
+    from pizza_amd import workloads as W
+    from pizza_amd.config import default_config
+    cfg = default_config(n_r_max=n_r, n_cheb_max=n_cheb, m_max=6, time_scheme=scheme, cheb_method="integ",
+                         matrix_solve="direct", buo_term=buo, dtMax=1.0e-6, ra=ra, raxi=raxi, sc=3.0, ek=1.0e-4, pr=1.0,
+                         radratio=0.35, l_ek_pump=pump)
+    print(f"case: integration m-loop n_r {n_r} {scheme}", flush=True)
+    seed = lambda x: W.seed_run(x, cfg, amp_t=1.0e-3, amp_xi=1.0e-3)  # noqa: E731
+    floors = _floor(cfg, [1, 6], seed)
+    g, o = _pair(cfg)
+    for x in (g, o):
+        seed(x)
+        x.start()
+    for i, n in enumerate((1, 5)):
+        g.step(n)
+        o.step(n)
+        for f in _fields(cfg):
+            err = rel(g.get_field(f), o.get_field(f))
+            assert err < max(1e-11, 10 * floors[i][f]), (f, i, err, floors[i][f])
