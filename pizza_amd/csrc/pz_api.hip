@@ -2275,30 +2275,39 @@ extern "C" int pz_time_series(pz_handle *h, pz_series *ts)
         const int N = h->N, nm = h->nm;
         const size_t F = (size_t)nm * N;
         std::memset(ts, 0, sizeof(*ts));
+        // the fields stay on the device: only their radial profiles, their
+        // m-spectra and the m = 0 columns come to the host
+        const int nchunk = (nm + PZ_PROF_M - 1) / PZ_PROF_M, np = PZ_NPROF * N;
+        std::vector<double> w(N); // pi r h dr of the spectra's integrals
+        for (int k = 0; k < N; k++) w[k] = rint_weights(h)[k] * (4.0 * std::atan(1.0)) * h->r[k] * h->height[k];
         cd *dd = nullptr;
-        double *dprof = nullptr, *dspec = nullptr;
+        double *dw = nullptr;
         HIPCHK(hipMallocAsync((void **)&dd, 2 * F * sizeof(cd), h->stream));
-        HIPCHK(hipMallocAsync((void **)&dprof, PZ_NPROF * (size_t)N * sizeof(double), h->stream));
-        HIPCHK(hipMallocAsync((void **)&dspec, 5 * F * sizeof(double), h->stream));
-        HIPCHK(hipMemsetAsync(dd, 0, 2 * F * sizeof(cd), h->stream));
+        HIPCHK(hipMallocAsync((void **)&dw, ((size_t)N + (size_t)(nchunk + 1) * np + 5 * (size_t)nm) * sizeof(double), h->stream));
+        double *dprof = dw + N, *dpart = dprof + np, *dspec = dpart + (size_t)nchunk * np;
+        HIPCHK(hipMemcpyAsync(dw, w.data(), N * sizeof(double), hipMemcpyHostToDevice, h->stream));
         series_derivatives(h, dd, dd + F);
-        hipLaunchKernelGGL(k_series_profiles, dim3((N + 63) / 64), dim3(64), 0, h->stream, h->d, (const cd *)dd,
-                           (const cd *)(dd + F), dprof);
-        hipLaunchKernelGGL(k_spectra_mr, dim3((int)((F + 255) / 256)), dim3(256), 0, h->stream, h->d, dspec);
+        hipLaunchKernelGGL(k_series_profiles, dim3((N + 63) / 64, nchunk), dim3(256), 0, h->stream, (const PzDev *)h->ddev,
+                           (const cd *)dd, (const cd *)(dd + F), dpart);
+        hipLaunchKernelGGL(k_series_finish, dim3((np + 63) / 64), dim3(64), 0, h->stream, (const double *)dpart, nchunk, np, dprof);
+        hipLaunchKernelGGL(k_spectra_m, dim3(nm), dim3(64), 0, h->stream, (const PzDev *)h->ddev, (const double *)dw, dspec);
         HIPCHK(hipGetLastError());
-        std::vector<double> prof(PZ_NPROF * (size_t)N), spec(5 * F);
-        std::vector<double2> dT(F), dX(F), T(F), X(F);
+        std::vector<double> prof(np), spec(5 * (size_t)nm);
+        std::vector<double2> dT(N), dX(N), T(N), X(N); // m = 0
         PzScheme s;
         HIPCHK(hipMemcpyAsync(prof.data(), dprof, prof.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipMemcpyAsync(spec.data(), dspec, spec.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(hipMemcpyAsync(dT.data(), dd, F * sizeof(cd), hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(hipMemcpyAsync(dX.data(), dd + F, F * sizeof(cd), hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(hipMemcpyAsync(T.data(), h->d.temp, F * sizeof(cd), hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(hipMemcpyAsync(X.data(), h->d.xi, F * sizeof(cd), hipMemcpyDeviceToHost, h->stream));
+        if (h->l_heat) {
+            HIPCHK(hipMemcpyAsync(dT.data(), dd, N * sizeof(cd), hipMemcpyDeviceToHost, h->stream));
+            HIPCHK(hipMemcpyAsync(T.data(), h->d.temp, N * sizeof(cd), hipMemcpyDeviceToHost, h->stream));
+        }
+        if (h->l_chem) {
+            HIPCHK(hipMemcpyAsync(dX.data(), dd + F, N * sizeof(cd), hipMemcpyDeviceToHost, h->stream));
+            HIPCHK(hipMemcpyAsync(X.data(), h->d.xi, N * sizeof(cd), hipMemcpyDeviceToHost, h->stream));
+        }
         HIPCHK(hipMemcpyAsync(&s, h->d.ss, sizeof(s), hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipFreeAsync(dd, h->stream));
-        HIPCHK(hipFreeAsync(dprof, h->stream));
-        HIPCHK(hipFreeAsync(dspec, h->stream));
+        HIPCHK(hipFreeAsync(dw, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
 
         const double pi = 4.0 * std::atan(1.0), tiny = 10.0 * 2.220446049250313e-16;
@@ -2308,14 +2317,19 @@ extern "C" int pz_time_series(pz_handle *h, pz_series *ts)
         const std::vector<double> us2 = row(0), up2 = row(1), upa = row(2), enst = row(3), buo = row(4), chem = row(5);
         std::vector<double> nuv = row(6), shv = row(7), flux = row(8);
         std::vector<double> rc(N), t(N);
-        // radial functions not kept on the host
-        HIPCHK(hipMemcpy(rc.data(), h->d.rgrav, N * sizeof(double), hipMemcpyDeviceToHost));
+        // radial functions not kept on the host, from the block of rows
+        std::vector<double> rows(PZ_NRADC * (size_t)N);
+        HIPCHK(hipMemcpy(rows.data(), h->d.radc, rows.size() * sizeof(double), hipMemcpyDeviceToHost));
+        const RadView R(rows.data(), N);
         std::vector<double> ekp(N), tcond(N), dtcond(N), xicond(N), dxicond(N);
-        HIPCHK(hipMemcpy(ekp.data(), h->d.ekpump, N * sizeof(double), hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(tcond.data(), h->d.tcond, N * sizeof(double), hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(dtcond.data(), h->d.dtcond, N * sizeof(double), hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(xicond.data(), h->d.xicond, N * sizeof(double), hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(dxicond.data(), h->d.dxicond, N * sizeof(double), hipMemcpyDeviceToHost));
+        for (int k = 0; k < N; k++) {
+            rc[k] = R.rgrav(k);
+            ekp[k] = R.ekpump(k);
+            tcond[k] = R.tcond(k);
+            dtcond[k] = R.dtcond(k);
+            xicond[k] = R.xicond(k);
+            dxicond[k] = R.dxicond(k);
+        }
         const double CorFac = h->d.CorFac, BuoFac = h->d.BuoFac, ChemFac = h->d.ChemFac, TdiffFac = h->d.TdiffFac;
         const double ViscFac = h->d.ViscFac;
         auto integ = [&](auto fn) {
@@ -2364,11 +2378,11 @@ extern "C" int pz_time_series(pz_handle *h, pz_series *ts)
         // length scales (get_lengthscales, :897-962; dl_diss, :694-701)
         std::vector<double> us2m(nm), up2m(nm), enm(nm), tm(nm), xm(nm);
         for (int i = 0; i < nm; i++) {
-            double a[5] = {0, 0, 0, 0, 0};
-            for (int j = 0; j < 5; j++)
-                for (int k = 0; k < N; k++)
-                    a[j] += rint_weights(h)[k] * (pi * spec[(size_t)j * F + (size_t)i * N + k] * r[k] * hg[k]);
-            us2m[i] = a[0]; up2m[i] = a[1]; enm[i] = a[2]; tm[i] = a[3]; xm[i] = a[4];
+            us2m[i] = spec[i];
+            up2m[i] = spec[nm + i];
+            enm[i] = spec[2 * (size_t)nm + i];
+            tm[i] = spec[3 * (size_t)nm + i];
+            xm[i] = spec[4 * (size_t)nm + i];
         }
         auto peak = [&](const std::vector<double> &v) {
             int best = -1;
@@ -2390,13 +2404,13 @@ extern "C" int pz_time_series(pz_handle *h, pz_series *ts)
             ts->lengths[4] = std::fabs(visc_2D) > tiny ? std::sqrt(2.0 * (us2_2D + up2_2D) * ViscFac / visc_2D) : 0.0;
         else
             ts->lengths[4] = std::fabs(visc_3D) > tiny ? std::sqrt(2.0 * (us2_3D + up2_3D) * ViscFac / visc_3D) : 0.0;
-        // heat and composition (:720-828), m = 0 at index 0
-        const int i0 = 0, mid = N / 2 - 1; // int(n_r_max/2), 1-based
+        // heat and composition (:720-828), the m = 0 columns
+        const int mid = N / 2 - 1; // int(n_r_max/2), 1-based
         if (h->l_heat) {
-            ts->heat[4] = ro(T[(size_t)i0 * N].x + tcond[0]);
-            ts->heat[5] = ro(T[(size_t)i0 * N + N - 1].x + tcond[N - 1]);
-            ts->heat[0] = ro(std::fabs(dtcond[0]) > tiny ? 1.0 + dT[(size_t)i0 * N].x / dtcond[0] : 1.0);
-            ts->heat[1] = ro(std::fabs(dtcond[N - 1]) > tiny ? 1.0 + dT[(size_t)i0 * N + N - 1].x / dtcond[N - 1] : 1.0);
+            ts->heat[4] = ro(T[0].x + tcond[0]);
+            ts->heat[5] = ro(T[N - 1].x + tcond[N - 1]);
+            ts->heat[0] = ro(std::fabs(dtcond[0]) > tiny ? 1.0 + dT[0].x / dtcond[0] : 1.0);
+            ts->heat[1] = ro(std::fabs(dtcond[N - 1]) > tiny ? 1.0 + dT[N - 1].x / dtcond[N - 1] : 1.0);
             for (int k = 0; k < N; k++) nuv[k] *= r[k] * hg[k];
             const double nv = rint_w(h, nuv);
             const double nc = integ([&](int k) { return dtcond[k] * dtcond[k] * hg[k] * r[k]; });
@@ -2415,18 +2429,18 @@ extern "C" int pz_time_series(pz_handle *h, pz_series *ts)
             } else {
                 ts->heat[3] = ro(simps_x(f2, th) / simps_x(f1, th));
             }
-            ts->heat[6] = ro(dtcond[mid] + dT[(size_t)i0 * N + mid].x);
+            ts->heat[6] = ro(dtcond[mid] + dT[mid].x);
         }
         if (h->l_chem) {
-            ts->chem[3] = ro(X[(size_t)i0 * N].x + xicond[0]);
-            ts->chem[4] = ro(X[(size_t)i0 * N + N - 1].x + xicond[N - 1]);
-            ts->chem[0] = ro(1.0 + dX[(size_t)i0 * N].x / dxicond[0]);
-            ts->chem[1] = ro(1.0 + dX[(size_t)i0 * N + N - 1].x / dxicond[N - 1]);
+            ts->chem[3] = ro(X[0].x + xicond[0]);
+            ts->chem[4] = ro(X[N - 1].x + xicond[N - 1]);
+            ts->chem[0] = ro(1.0 + dX[0].x / dxicond[0]);
+            ts->chem[1] = ro(1.0 + dX[N - 1].x / dxicond[N - 1]);
             for (int k = 0; k < N; k++) shv[k] *= r[k] * hg[k];
             const double sv = rint_w(h, shv);
             const double sc = integ([&](int k) { return dxicond[k] * dxicond[k] * hg[k] * r[k]; });
             ts->chem[2] = ro(1.0 + sv / sc);
-            ts->chem[5] = ro(dxicond[mid] + dX[(size_t)i0 * N + mid].x);
+            ts->chem[5] = ro(dxicond[mid] + dX[mid].x);
         }
         if (h->c.l_non_rot) {
             // a non-rotating run writes no 3D series (outputs.f90:102-121)

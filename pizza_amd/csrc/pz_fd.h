@@ -651,7 +651,7 @@ __device__ __forceinline__ void fd_mloop_body(const PzDev &p, int mi, int istage
         if (m == 0) { gP[0] = z; gP[N + 1] = z; }
         else { gP[0] = z; gP[1] = z; gP[N + 2] = z; gP[N + 3] = z; }
     }
-    __syncthreads();
+    lds_barrier();
     // the solves, one wave each (blocks of 256 threads)
     const int wave = tid >> 6;
     if (wave == 0 && hT) fd_tri_solve_wave(N, mT, mT + N, mT + 2 * N, gT);
@@ -660,13 +660,13 @@ __device__ __forceinline__ void fd_mloop_body(const PzDev &p, int mi, int istage
         if (m == 0) fd_tri_solve_wave(N, (const double *)mP, (const double *)mP + N, (const double *)mP + 2 * N, gP);
         else fd_penta_solve_wave(N, mP, mP + N, mP + 2 * N, mP + 3 * N, mP + 4 * N, gP);
     }
-    __syncthreads();
+    lds_barrier();
     if (tid == 0) {
         if (hT) fd_ghost_scalar(gT, N, p.ktopt, p.kbott, R, fd_wall(p, p.topt, mi), fd_wall(p, p.bott, mi));
         if (hX) fd_ghost_scalar(gX, N, p.ktopxi, p.kbotxi, R, fd_wall(p, p.topxi, mi), fd_wall(p, p.botxi, mi));
         fd_ghost_psi(p, R, m, gP);
     }
-    __syncthreads();
+    lds_barrier();
     const int inext = (istage == p.nstages) ? 1 : istage + 1;
     // implicit terms for the next stage; also before a CNAB2 start-up step
     const int lcalc = p.l_imp_calc_rhs[inext - 1] || (p.bridge && ss->n_steps + 1 <= p.nold - 1);
@@ -751,54 +751,81 @@ __device__ __forceinline__ double cc22r(cd a, cd b, int m)
     return m == 0 ? a.x * b.x : 2.0 * (a.x * b.x + a.y * b.y);
 }
 
-// Radial profiles of get_time_series (outputs.f90:456-502), one thread per
-// radius: out[j * N + r] for j = us2, up2, up2_axi, enstrophy, buoyancy
-// power, chemical power, volume Nusselt and Sherwood integrands (before
-// the r h factor), radial heat flux.
+// Radial profiles of get_time_series (outputs.f90:456-502): j = us2, up2,
+// up2_axi, enstrophy, buoyancy power, chemical power, volume Nusselt and
+// Sherwood integrands (before the r h factor), radial heat flux.  Bound by
+// the reads of the fields, so the modes are split over workgroups of 64 radii
+// by PZ_PROF_M modes (four per thread, coalesced along the radius) whose sums
+// go to part[chunk][j][N]; k_series_finish adds the chunks.  One thread per
+// radius over all modes took 481 us at n_r 257 with 683 modes.
 #define PZ_NPROF 9
-__global__ void k_series_profiles(const PzDev p __attribute__((grid_constant)), const cd *dT, const cd *dX, double *out)
+#define PZ_PROF_M 16
+__global__ void __launch_bounds__(256) k_series_profiles(const PzDev *__restrict__ pd, const cd *dT, const cd *dX, double *part)
 {
-    const int nr = blockIdx.x * blockDim.x + threadIdx.x;
-    if (nr >= p.N) return;
-    const int N = p.N;
+    const PzDev &p = *pd;
+    __shared__ double acc[3][PZ_NPROF][64];
+    const int N = p.N, lane = threadIdx.x & 63, sub = threadIdx.x >> 6, nr = blockIdx.x * 64 + lane;
     double v[PZ_NPROF] = {};
-    const double o2 = p.or2[nr];
-    for (int i = 0; i < p.nm; i++) {
-        const int m = p.idx2m[i];
-        const size_t q = (size_t)i * N + nr;
-        const cd us = p.us[q];
-        v[0] += cc2r(us, m);
-        v[1] += cc2r(p.up[q], m);
-        v[2] += m == 0 ? cc2r(p.up[q], m) : 0.0;
-        v[3] += cc2r(p.om[q], m);
-        if (p.l_heat) {
-            const cd t = p.temp[q];
-            v[4] += cc22r(us, t, m);
-            v[6] += cc2r(dT[q], m) + (double)m * (double)m * o2 * cc2r(t, m);
-            v[8] += cc22r(us, t, m);
-            if (m == 0) v[8] += -p.TdiffFac * dT[q].x - p.TdiffFac * p.dtcond[nr];
-        }
-        if (p.l_chem) {
-            const cd x = p.xi[q];
-            v[5] += cc22r(us, x, m);
-            v[7] += cc2r(dX[q], m) + (double)m * (double)m * o2 * cc2r(x, m);
+    if (nr < N) {
+        const double o2 = p.or2[nr];
+        for (int i = blockIdx.y * PZ_PROF_M + sub; i < min(p.nm, (int)(blockIdx.y + 1) * PZ_PROF_M); i += 4) {
+            const int m = p.idx2m[i];
+            const size_t q = (size_t)i * N + nr;
+            const cd us = p.us[q], up = p.up[q];
+            v[0] += cc2r(us, m);
+            v[1] += cc2r(up, m);
+            v[2] += m == 0 ? cc2r(up, m) : 0.0;
+            v[3] += cc2r(p.om[q], m);
+            if (p.l_heat) {
+                const cd t = p.temp[q], d = dT[q];
+                v[4] += cc22r(us, t, m);
+                v[6] += cc2r(d, m) + (double)m * (double)m * o2 * cc2r(t, m);
+                v[8] += cc22r(us, t, m);
+                if (m == 0) v[8] += -p.TdiffFac * d.x - p.TdiffFac * p.dtcond[nr];
+            }
+            if (p.l_chem) {
+                const cd x = p.xi[q];
+                v[5] += cc22r(us, x, m);
+                v[7] += cc2r(dX[q], m) + (double)m * (double)m * o2 * cc2r(x, m);
+            }
         }
     }
-    for (int j = 0; j < PZ_NPROF; j++) out[(size_t)j * N + nr] = v[j];
+    if (sub > 0)
+        for (int j = 0; j < PZ_NPROF; j++) acc[sub - 1][j][lane] = v[j];
+    __syncthreads();
+    if (sub == 0 && nr < N)
+        for (int j = 0; j < PZ_NPROF; j++)
+            part[((size_t)blockIdx.y * PZ_NPROF + j) * N + nr] = ((v[j] + acc[0][j][lane]) + acc[1][j][lane]) + acc[2][j][lane];
+}
+// out[i] = sum over nchunk of part[chunk][n], one thread each
+__global__ void __launch_bounds__(64) k_series_finish(const double *part, int nchunk, int n, double *out)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double s = 0.0;
+    for (int c = 0; c < nchunk; c++) s += part[(size_t)c * n + i];
+    out[i] = s;
 }
 
-// Per (m, r) squares of calculate_spectra (spectra.f90:131-153) before the
-// pi r h factor and the radial integral: out[(j * nm + i) * N + r] for
-// j = us, up, omega, T, xi.
-__global__ void k_spectra_mr(const PzDev p __attribute__((grid_constant)), double *out)
+// The m-spectra of calculate_spectra (spectra.f90:131-153): the radial
+// integrals (weights w, with the pi r h factor) of |u_s|^2, |u_phi|^2,
+// |omega|^2, |T|^2 and |xi|^2, one wave per mode: out[j * nm + i].
+__global__ void __launch_bounds__(64) k_spectra_m(const PzDev *__restrict__ pd, const double *w, double *out)
 {
-    const size_t F = (size_t)p.nm * p.N;
-    const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= F) return;
-    const int m = p.idx2m[q / p.N];
-    out[q] = cc2r(p.us[q], m);
-    out[F + q] = cc2r(p.up[q], m);
-    out[2 * F + q] = cc2r(p.om[q], m);
-    out[3 * F + q] = p.l_heat ? cc2r(p.temp[q], m) : 0.0;
-    out[4 * F + q] = p.l_chem ? cc2r(p.xi[q], m) : 0.0;
+    const PzDev &p = *pd;
+    const int N = p.N, i = blockIdx.x, m = p.idx2m[i];
+    double a[5] = {};
+    for (int k = threadIdx.x; k < N; k += 64) {
+        const size_t q = (size_t)i * N + k;
+        const double wk = w[k];
+        a[0] += wk * cc2r(p.us[q], m);
+        a[1] += wk * cc2r(p.up[q], m);
+        a[2] += wk * cc2r(p.om[q], m);
+        if (p.l_heat) a[3] += wk * cc2r(p.temp[q], m);
+        if (p.l_chem) a[4] += wk * cc2r(p.xi[q], m);
+    }
+    for (int j = 0; j < 5; j++) {
+        const double s = wave_sum(a[j]);
+        if (threadIdx.x == 0) out[(size_t)j * p.nm + i] = s;
+    }
 }
