@@ -932,8 +932,7 @@ static void allow_full_lds(int lim)
                              (const void *)k_start, (const void *)k_build_inv, (const void *)k_mcoll,
                              (const void *)k_start_coll, (const void *)k_build_lhs_batch,
                              (const void *)k_mphase_batch, (const void *)k_mphase_batch_small, (const void *)k_radial_loop_batch,
-                             (const void *)k_build_inv_batch, (const void *)k_mcoll_batch<true>, (const void *)k_mcoll_batch<false>, (const void *)k_fd_build,
-                             (const void *)k_fd_mloop, (const void *)k_fd_start, (const void *)k_radial_loop_big,
+                             (const void *)k_build_inv_batch, (const void *)k_mcoll_batch<true>, (const void *)k_mcoll_batch<false>,                              (const void *)k_fd_mloop, (const void *)k_fd_start, (const void *)k_radial_loop_big,
                              (const void *)k_radial_loop_inplace,
                              (const void *)k_adj_probe, (const void *)k_mcoll_adj, (const void *)k_radial_adj,
                              (const void *)k_start_coll_adj, (const void *)k_assemble_coll,
@@ -1201,6 +1200,12 @@ static void setup(pz_handle *h)
     d.dVsT = h->dalloc<cd>(F); d.dVsXi = h->dalloc<cd>(F); d.dVsOm = h->dalloc<cd>(F);
     d.dtr = h->dalloc<double>(N);
     d.dth = h->dalloc<double>(N);
+    {
+        unsigned long long big;
+        const double lim = 1.0e300;
+        std::memcpy(&big, &lim, sizeof(big));
+        d.cacc = h->upload(std::vector<unsigned long long>{big, big, 0ull});
+    }
     // factorised matrices
     const int nm = h->nm, nb2 = N - 2;
     d.T_A1 = h->dalloc<double>(nm * 4); d.T_A2 = h->dalloc<double>((size_t)nm * 2 * nb2);
@@ -1928,9 +1933,11 @@ static void launch_radial(pz_handle *h, int is, int courant)
                            (const PzDev *)h->ddev, is, courant);
     }
 }
-static void launch_explicit(pz_handle *h, int stage)
+// stage 1 evaluates the Courant limits; with decide, its last workgroup also
+// takes the decision of launch_courant
+static void launch_explicit(pz_handle *h, int stage, bool decide = false)
 {
-    if (h->sch.l_exp_calc[stage - 1]) launch_radial(h, stage - 1, stage == 1 ? 1 : 0);
+    if (h->sch.l_exp_calc[stage - 1]) launch_radial(h, stage - 1, stage != 1 ? 0 : decide ? 2 : 1);
 }
 
 // Stage 1: dt_courant, the dt roll, set_weights and the rebuild flag
@@ -1950,7 +1957,7 @@ __global__ void k_force_lmat(PzScheme *s)
 static void launch_builds(pz_handle *h)
 {
     if (h->d.fd) {
-        hipLaunchKernelGGL(k_fd_build, dim3(h->nm), dim3(256), h->lds_fd, h->stream, (const PzDev *)h->ddev, 0);
+        // k_fd_mloop rebuilds its mode's systems itself at stage 1
     } else if (h->d.coll) {
         hipLaunchKernelGGL(k_build_coll, dim3(h->nm, h->d.dmat ? 4 : 3), dim3(1024), h->lds_gj, h->stream,
                            (const PzDev *)h->ddev, 0);
@@ -1995,9 +2002,9 @@ static void launch_implicit(pz_handle *h, int stage)
 static void launch_step(pz_handle *h)
 {
     for (int stage = 1; stage <= h->sch.nstages; stage++) {
-        launch_explicit(h, stage);
+        launch_explicit(h, stage, true);
         if (stage == 1) {
-            launch_courant(h);
+            if (!h->sch.l_exp_calc[0]) launch_courant(h);
             launch_builds(h);
         }
         launch_implicit(h, stage);
@@ -3121,9 +3128,10 @@ static void launch_class_step(const pz_ensemble *e, const EnsClass &c)
         const int exp_calc = s.l_exp_calc[stage - 1];
         if (exp_calc)
             hipLaunchKernelGGL(k_radial_loop_batch, dim3(c.nb_r), dim3(256), c.lds_r, c.stream,
-                               PzBatch{runs, c.map_r, (int)c.members.size()}, stage - 1, stage == 1 ? 1 : 0);
+                               PzBatch{runs, c.map_r, (int)c.members.size()}, stage - 1, stage == 1 ? 2 : 0);
         if (stage == 1) {
-            hipLaunchKernelGGL(k_courant_batch, dim3(c.nb_c), dim3(256), 0, c.stream, PzBatch{runs, c.map_c, (int)c.members.size()});
+            if (!exp_calc)
+                hipLaunchKernelGGL(k_courant_batch, dim3(c.nb_c), dim3(256), 0, c.stream, PzBatch{runs, c.map_c, (int)c.members.size()});
             if (e->coll) {
                 hipLaunchKernelGGL(k_build_coll_batch, dim3(std::min(c.nb_3, 512)), dim3(1024), c.lds_gj, c.stream,
                                    PzBatch{runs, c.map_3, (int)c.members.size()}, c.nb_3, 0);

@@ -666,504 +666,6 @@ __device__ double block_reduce(double v, double *scratch, int op /*0 sum, 1 max*
 }
 
 // ---------------------------------------------------------------------------
-// Radial loop: rloop::radial_loop (radial_loop.f90:264-392) for one radius
-// per workgroup.  Real fields travel in pairs through one complex FFT.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ void radial_loop_body(const PzDev &p, int nr, int is, int courant)
-{
-    extern __shared__ double smem[];
-    const int n = p.nphi, nm = p.nm, N = p.N;
-    const size_t F = (size_t)nm * N;
-    cd *spec = (cd *)smem;           // 5 x nm
-    cd *bufa = spec + 5 * nm;        // 3 x n
-    cd *bufb = bufa + 3 * n;         // 3 x n
-    cd *twl = bufb + 3 * n;          // n twiddles exp(-2 pi i k / n)
-    double *red = (double *)(twl + n);
-    const int nin = (p.l_heat || p.l_chem) ? (p.l_chem ? 3 : 2) : 2;
-
-    for (int k = threadIdx.x; k < n; k += blockDim.x) twl[k] = p.twid[k];
-    for (int i = threadIdx.x; i < nm; i += blockDim.x) {
-        size_t q = (size_t)i * N + nr;
-        spec[i] = p.us[q];
-        spec[nm + i] = p.up[q];
-        spec[2 * nm + i] = p.om[q];
-        spec[3 * nm + i] = p.l_heat ? p.temp[q] : mk(0, 0);
-        spec[4 * nm + i] = p.l_chem ? p.xi[q] : mk(0, 0);
-    }
-    lds_barrier();
-    // Reynolds-stress m-sum (radial_loop.f90:267-278)
-    double part = 0.0;
-    for (int i = threadIdx.x; i < nm; i += blockDim.x) {
-        int m = p.idx2m[i];
-        cd usf = m == 0 ? cscale(0.5 * p.ek * p.CorFac * p.ekpump[nr], spec[nm + i]) : spec[i];
-        part += cc22real(usf, spec[2 * nm + i], m);
-    }
-    double usom = block_reduce(part, red, 0);
-    // pairs (us,up), (om,T), (xi,0) as Hermitian spectra of z = a + i b
-    auto packed = [=](int tr, int k) {
-        // a + i b from the m < n_m half, its conjugate from the other
-        const bool lo = k < nm, hi = !lo && n - k < nm;
-        const int kk = lo ? k : n - k;
-        if (!lo && !hi) return mk(0.0, 0.0);
-        const cd a = spec[(2 * tr) * nm + kk];
-        const cd b = (2 * tr + 1) < 5 ? spec[(2 * tr + 1) * nm + kk] : mk(0.0, 0.0);
-        if (k == 0) return mk(a.x, b.x);
-        return lo ? mk(a.x - b.y, a.y + b.x) : mk(a.x + b.y, b.x - a.y);
-    };
-    // register FFTs (one wave per transform, packing as they load) where
-    // n_phi = 64 P, else LDS Stockham FFTs of the packed columns
-    const int Pw = wave_fft_p_phi(n);
-    cd *g;
-    if (Pw) {
-        fft_wave_phi(Pw, nin, packed, [=](int tr, int k, cd v) { bufb[tr * n + k] = v; },
-                     [=](int k) { const cd w = twl[k]; return mk(w.x, -w.y); });
-        lds_barrier();
-        g = bufb;
-    } else {
-        for (int t = threadIdx.x; t < nin * n; t += blockDim.x) {
-            const int tr = t / n;
-            bufa[t] = packed(tr, t - tr * n);
-        }
-        lds_barrier();
-        g = fft_stockham(bufa, bufb, n, nin, +1, p.radices, p.nrad,
-                         [&](int k) { const cd w = twl[k]; return mk(w.x, -w.y); });
-    }
-    cd *o = (g == bufa) ? bufb : bufa;
-    // Courant (courant.f90:41-76)
-    if (courant) {
-        double vr = 0.0, vh = 0.0;
-        for (int j = threadIdx.x; j < n; j += blockDim.x) {
-            cd z = g[j];
-            vr = fmax(vr, z.x * z.x);
-            vh = fmax(vh, z.y * z.y);
-        }
-        vr = block_reduce(vr, red, 1);
-        vh = block_reduce(vh, red, 1);
-        if (threadIdx.x == 0) {
-            double cf = p.courfac;
-            vr = cf * cf * vr;
-            vh = cf * cf * vh;
-            double dtrk = 1.0e10, dthk = 1.0e10;
-            if (vr != 0.0) dtrk = fmin(dtrk, sqrt(p.delxr2[nr] / vr));
-            if (vh != 0.0) dthk = fmin(dthk, sqrt(p.delxh2[nr] / vh));
-            p.dtr[nr] = dtrk;
-            p.dth[nr] = dthk;
-        }
-    }
-    // nonlinear products (radial_loop.f90:316-325): (upX + i r us X)
-    const double rr = p.r[nr];
-    const int nout = 1 + (p.l_heat ? 1 : 0) + (p.l_chem ? 1 : 0); // omega, then T and xi as present
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-        cd z0 = g[j], z1 = g[n + j];
-        double us = z0.x, up = z0.y, om = z1.x, T = z1.y;
-        o[j] = mk(up * om, rr * us * om);
-        if (p.l_heat) o[n + j] = mk(up * T, rr * us * T);
-        if (p.l_chem) {
-            double X = g[2 * n + j].x;
-            o[(p.l_heat ? 2 : 1) * n + j] = mk(up * X, rr * us * X);
-        }
-    }
-    lds_barrier();
-    cd *other = (o == bufa) ? bufb : bufa;
-    cd *Z;
-    if (Pw) {
-        fft_wave_phi(Pw, nout, [=](int tr, int i) { return o[tr * n + i]; },
-                     [=](int tr, int k, cd v) { other[tr * n + k] = v; }, [=](int k) { return twl[k]; });
-        lds_barrier();
-        Z = other;
-    } else {
-        Z = fft_stockham(o, other, n, nout, -1, p.radices, p.nrad, [&](int k) { return twl[k]; });
-    }
-    // unpack, normalise and post-scale (radial_loop.f90:350-386)
-    const double or1 = p.or1[nr];
-    const double fbeta = (1.0 - p.tadvz) * p.beta[nr] * or1;
-    for (int t = threadIdx.x; t < nout * nm; t += blockDim.x) {
-        int tr = t / nm, i = t - tr * nm;
-        cd zk = Z[tr * n + i], zc = cconj(Z[tr * n + (i == 0 ? 0 : n - i)]);
-        cd A = mk(0.5 * (zk.x + zc.x), 0.5 * (zk.y + zc.y));  // spectrum of up*X
-        cd B = mk(0.5 * (zk.y - zc.y), -0.5 * (zk.x - zc.x)); // spectrum of r us X
-        A = cdivr(A, (double)n);
-        B = cdivr(B, (double)n);
-        int m = p.idx2m[i];
-        size_t q = (size_t)i * N + nr;
-        cd cim = mk(0.0, -or1 * (double)m); // -or1*ci*m
-        if (tr == 0) {
-            p.P_expl[is * F + q] = (i == 0) ? mk(-usom, 0.0) : cmul(cim, A);
-            p.dVsOm[q] = B;
-        } else if (tr == 1 && p.l_heat) {
-            cd v = cmul(cim, A);
-            p.T_expl[is * F + q] = mk(v.x - fbeta * B.x, v.y - fbeta * B.y);
-            p.dVsT[q] = B;
-        } else {
-            p.X_expl[is * F + q] = cmul(cim, A);
-            p.dVsXi[q] = B;
-        }
-    }
-}
-
-// The radial loop for long azimuthal grids (n_phi too large for the staged
-// variant above): the spectra are packed straight from global memory and
-// the real fields travel through the complex FFTs one pair at a time, so
-// LDS holds four columns of n_phi values (three fields and one scratch).
-__device__ __forceinline__ void radial_loop_big_body(const PzDev &p, int nr, int is, int courant)
-{
-    extern __shared__ double smem[];
-    const int n = p.nphi, nm = p.nm, N = p.N;
-    const size_t F = (size_t)nm * N;
-    cd *s0 = (cd *)smem, *s1 = s0 + n, *s2 = s1 + n, *sc = s2 + n;
-    double *red = (double *)(sc + n);
-    // without composition the third column holds the twiddle table
-    const bool twl_lds = !p.l_chem;
-    cd *twl = s2;
-    if (twl_lds)
-        for (int k = threadIdx.x; k < n; k += blockDim.x) twl[k] = p.twid[k];
-    auto fwd = [&](int k) { return twl_lds ? twl[k] : p.twid[k]; };
-    auto bwd = [&](int k) {
-        const cd w = twl_lds ? twl[k] : p.twid[k];
-        return mk(w.x, -w.y);
-    };
-    // Reynolds-stress m-sum (radial_loop.f90:267-278)
-    double part = 0.0;
-    for (int i = threadIdx.x; i < nm; i += blockDim.x) {
-        const int m = p.idx2m[i];
-        const size_t q = (size_t)i * N + nr;
-        const cd usf = m == 0 ? cscale(0.5 * p.ek * p.CorFac * p.ekpump[nr], p.up[q]) : p.us[q];
-        part += cc22real(usf, p.om[q], m);
-    }
-    const double usom = block_reduce(part, red, 0);
-    // Hermitian spectra of z = a + i b for (us, up), (om, T), (xi, 0)
-    for (int t = threadIdx.x; t < 3 * n; t += blockDim.x) {
-        const int tr = t / n, k = t - tr * n;
-        if (tr == 2 && !p.l_chem) break;
-        const cd *A = tr == 0 ? p.us : (tr == 1 ? p.om : p.xi);
-        const cd *B = tr == 0 ? p.up : (tr == 1 ? (p.l_heat ? p.temp : nullptr) : nullptr);
-        cd z = mk(0, 0);
-        if (k == 0) {
-            z = mk(A[nr].x, B ? B[nr].x : 0.0);
-        } else if (k < nm) {
-            const cd a = A[(size_t)k * N + nr], b = B ? B[(size_t)k * N + nr] : mk(0, 0);
-            z = mk(a.x - b.y, a.y + b.x);
-        } else if (n - k < nm) {
-            const int kk = n - k;
-            const cd a = cconj(A[(size_t)kk * N + nr]), b = B ? cconj(B[(size_t)kk * N + nr]) : mk(0, 0);
-            z = mk(a.x - b.y, a.y + b.x);
-        }
-        (tr == 0 ? s0 : (tr == 1 ? s1 : s2))[k] = z;
-    }
-    lds_barrier();
-    // one complex FFT at a time; the result lands in the column or in the
-    // scratch, whose roles are then exchanged
-    {
-        cd *g = fft_stockham(s0, sc, n, 1, +1, p.radices, p.nrad, bwd);
-        if (g != s0) { sc = s0; s0 = g; }
-        lds_barrier();
-        g = fft_stockham(s1, sc, n, 1, +1, p.radices, p.nrad, bwd);
-        if (g != s1) { sc = s1; s1 = g; }
-        if (p.l_chem) {
-            lds_barrier();
-            g = fft_stockham(s2, sc, n, 1, +1, p.radices, p.nrad, bwd);
-            if (g != s2) { sc = s2; s2 = g; }
-        }
-        lds_barrier();
-    }
-    if (courant) {
-        double vr = 0.0, vh = 0.0;
-        for (int j = threadIdx.x; j < n; j += blockDim.x) {
-            const cd z = s0[j];
-            vr = fmax(vr, z.x * z.x);
-            vh = fmax(vh, z.y * z.y);
-        }
-        vr = block_reduce(vr, red, 1);
-        vh = block_reduce(vh, red, 1);
-        if (threadIdx.x == 0) {
-            const double cf = p.courfac;
-            vr = cf * cf * vr;
-            vh = cf * cf * vh;
-            double dtrk = 1.0e10, dthk = 1.0e10;
-            if (vr != 0.0) dtrk = fmin(dtrk, sqrt(p.delxr2[nr] / vr));
-            if (vh != 0.0) dthk = fmin(dthk, sqrt(p.delxh2[nr] / vh));
-            p.dtr[nr] = dtrk;
-            p.dth[nr] = dthk;
-        }
-    }
-    // nonlinear products in place (radial_loop.f90:316-325): (up X + i r us X)
-    const double rr = p.r[nr];
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-        const cd z0 = s0[j], z1 = s1[j];
-        const double us = z0.x, up = z0.y, om = z1.x, T = z1.y;
-        const double X = p.l_chem ? s2[j].x : 0.0;
-        s0[j] = mk(up * om, rr * us * om);
-        s1[j] = mk(up * T, rr * us * T);
-        if (p.l_chem) s2[j] = mk(up * X, rr * us * X);
-    }
-    lds_barrier();
-    {
-        cd *g = fft_stockham(s0, sc, n, 1, -1, p.radices, p.nrad, fwd);
-        if (g != s0) { sc = s0; s0 = g; }
-        if (p.l_heat) {
-            lds_barrier();
-            g = fft_stockham(s1, sc, n, 1, -1, p.radices, p.nrad, fwd);
-            if (g != s1) { sc = s1; s1 = g; }
-        }
-        if (p.l_chem) {
-            lds_barrier();
-            g = fft_stockham(s2, sc, n, 1, -1, p.radices, p.nrad, fwd);
-            if (g != s2) { sc = s2; s2 = g; }
-        }
-        lds_barrier();
-    }
-    // unpack, normalise and post-scale (radial_loop.f90:350-386)
-    const double or1 = p.or1[nr];
-    const double fbeta = (1.0 - p.tadvz) * p.beta[nr] * or1;
-    for (int t = threadIdx.x; t < 3 * nm; t += blockDim.x) {
-        const int tr = t / nm, i = t - tr * nm;
-        if ((tr == 1 && !p.l_heat) || (tr == 2 && !p.l_chem)) continue;
-        const cd *Z = tr == 0 ? s0 : (tr == 1 ? s1 : s2);
-        const cd zk = Z[i], zc = cconj(Z[i == 0 ? 0 : n - i]);
-        cd A = mk(0.5 * (zk.x + zc.x), 0.5 * (zk.y + zc.y));
-        cd B = mk(0.5 * (zk.y - zc.y), -0.5 * (zk.x - zc.x));
-        A = cdivr(A, (double)n);
-        B = cdivr(B, (double)n);
-        const int m = p.idx2m[i];
-        const size_t q = (size_t)i * N + nr;
-        const cd cim = mk(0.0, -or1 * (double)m);
-        if (tr == 0) {
-            p.P_expl[is * F + q] = (i == 0) ? mk(-usom, 0.0) : cmul(cim, A);
-            p.dVsOm[q] = B;
-        } else if (tr == 1) {
-            const cd v = cmul(cim, A);
-            p.T_expl[is * F + q] = mk(v.x - fbeta * B.x, v.y - fbeta * B.y);
-            p.dVsT[q] = B;
-        } else {
-            p.X_expl[is * F + q] = cmul(cim, A);
-            p.dVsXi[q] = B;
-        }
-    }
-}
-
-// Long azimuthal grids without composition, where two columns of n_phi and
-// the in-place transforms fit (fft_inplace_fits): the spectra by radius
-// come from k_gather_r (contiguous rows), the pairs (u_s, u_phi) and
-// (omega, T) travel through their in-place complex FFTs together, and LDS
-// holds the two columns and a two-level twiddle table (64 + n_phi / 64
-// entries).
-__device__ __forceinline__ void radial_loop_inplace_body(const PzDev &p, int nr, int is, int courant)
-{
-    extern __shared__ double smem[];
-    const int n = p.nphi, nm = p.nm, N = p.N;
-    const size_t F = (size_t)nm * N;
-    cd *s0 = (cd *)smem, *s1 = s0 + n, *t1 = s1 + n, *t2 = t1 + 64;
-    const int n2 = (n + 63) >> 6;
-    cd *om = t2 + n2;
-    double *red = (double *)(om + PZ_FFT_OM_MAX), *msr = red + 16;
-    const cd *Rus = p.rrow + (size_t)nr * nm, *Rup = Rus + F, *Rom = Rus + 2 * F, *RT = Rus + 3 * F;
-    // exp(-2 pi i k / n) = t1[k mod 64] t2[k / 64]
-    for (int k = threadIdx.x; k < 64 + n2; k += blockDim.x) t1[k] = p.twid[k < 64 ? k : 64 * (k - 64)];
-    auto fwd = [=](int k) { return cmul(t1[k & 63], t2[k >> 6]); };
-    auto bwd = [=](int k) {
-        const cd w = cmul(t1[k & 63], t2[k >> 6]);
-        return mk(w.x, -w.y);
-    };
-    // Hermitian spectra of z = a + i b for (us, up), (om, T), and the
-    // Reynolds-stress m-sum (radial_loop.f90:267-278) from the same loads,
-    // one partial sum per wave in msr (added at the unpack)
-    const double ekc = 0.5 * p.ek * p.CorFac * p.ekpump[nr];
-    double part = 0.0;
-    for (int k = threadIdx.x; k < n; k += blockDim.x) {
-        cd z0 = mk(0, 0), z1 = mk(0, 0);
-        if (k < nm) {
-            const cd us = Rus[k], up = Rup[k], o = Rom[k], T = p.l_heat ? RT[k] : mk(0, 0);
-            const int m = p.idx2m[k];
-            part += cc22real(m == 0 ? cscale(ekc, up) : us, o, m);
-            if (k == 0) {
-                z0 = mk(us.x, up.x);
-                z1 = mk(o.x, T.x);
-            } else {
-                z0 = mk(us.x - up.y, us.y + up.x);
-                z1 = mk(o.x - T.y, o.y + T.x);
-            }
-        } else if (n - k < nm) {
-            const int kk = n - k;
-            const cd us = cconj(Rus[kk]), up = cconj(Rup[kk]), o = cconj(Rom[kk]);
-            const cd T = p.l_heat ? cconj(RT[kk]) : mk(0, 0);
-            z0 = mk(us.x - up.y, us.y + up.x);
-            z1 = mk(o.x - T.y, o.y + T.x);
-        }
-        s0[k] = z0;
-        s1[k] = z1;
-    }
-    for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
-    if ((threadIdx.x & 63) == 0) msr[threadIdx.x >> 6] = part;
-    lds_barrier();
-    fft_inplace(s0, n, 2, +1, p.radices, p.nrad, bwd, om);
-    if (courant) {
-        double vr = 0.0, vh = 0.0;
-        for (int j = threadIdx.x; j < n; j += blockDim.x) {
-            const cd z = s0[j];
-            vr = fmax(vr, z.x * z.x);
-            vh = fmax(vh, z.y * z.y);
-        }
-        vr = block_reduce(vr, red, 1);
-        vh = block_reduce(vh, red, 1);
-        if (threadIdx.x == 0) {
-            const double cf = p.courfac;
-            vr = cf * cf * vr;
-            vh = cf * cf * vh;
-            double dtrk = 1.0e10, dthk = 1.0e10;
-            if (vr != 0.0) dtrk = fmin(dtrk, sqrt(p.delxr2[nr] / vr));
-            if (vh != 0.0) dthk = fmin(dthk, sqrt(p.delxh2[nr] / vh));
-            p.dtr[nr] = dtrk;
-            p.dth[nr] = dthk;
-        }
-    }
-    // nonlinear products in place (radial_loop.f90:316-325): (up X + i r us X)
-    const double rr = p.r[nr];
-    for (int j = threadIdx.x; j < n; j += blockDim.x) {
-        const cd z0 = s0[j], z1 = s1[j];
-        const double us = z0.x, up = z0.y, om = z1.x, T = z1.y;
-        s0[j] = mk(up * om, rr * us * om);
-        s1[j] = mk(up * T, rr * us * T);
-    }
-    lds_barrier();
-    fft_inplace(s0, n, p.l_heat ? 2 : 1, -1, p.radices, p.nrad, fwd, om);
-    // unpack, normalise and post-scale (radial_loop.f90:350-386)
-    const double or1 = p.or1[nr];
-    const double fbeta = (1.0 - p.tadvz) * p.beta[nr] * or1;
-    const int nout = p.l_heat ? 2 : 1;
-    for (int t = threadIdx.x; t < nout * nm; t += blockDim.x) {
-        const int tr = t >= nm, i = t - tr * nm;
-        const cd *Z = tr == 0 ? s0 : s1;
-        const cd zk = Z[i], zc = cconj(Z[i == 0 ? 0 : n - i]);
-        cd A = mk(0.5 * (zk.x + zc.x), 0.5 * (zk.y + zc.y));
-        cd B = mk(0.5 * (zk.y - zc.y), -0.5 * (zk.x - zc.x));
-        A = cdivr(A, (double)n);
-        B = cdivr(B, (double)n);
-        const int m = p.idx2m[i];
-        const size_t q = (size_t)i * N + nr;
-        const cd cim = mk(0.0, -or1 * (double)m);
-        if (tr == 0) {
-            if (i == 0) {
-                double usom = msr[0];
-                for (int w = 1; w < (int)((blockDim.x + 63) >> 6); w++) usom += msr[w];
-                p.P_expl[is * F + q] = mk(-usom, 0.0);
-            } else {
-                p.P_expl[is * F + q] = cmul(cim, A);
-            }
-            p.dVsOm[q] = B;
-        } else {
-            const cd v = cmul(cim, A);
-            p.T_expl[is * F + q] = mk(v.x - fbeta * B.x, v.y - fbeta * B.y);
-            p.dVsT[q] = B;
-        }
-    }
-}
-
-// u_s, u_phi, omega (and T) from the mode-major layout [m][n_r] to rows by
-// radius [f][n_r][n_m]: 16 x 32 tiles of all fields through LDS, coalesced
-// on both sides, every load of a thread in flight before the one barrier
-#define PZ_GATHER_TM 16
-#define PZ_GATHER_TR 32
-__global__ void __launch_bounds__(256) k_gather_r(const PzDev *__restrict__ pd)
-{
-    const PzDev &p = *pd;
-    __shared__ cd tile[4][PZ_GATHER_TM][PZ_GATHER_TR + 1];
-    const int N = p.N, nm = p.nm;
-    const size_t F = (size_t)nm * N;
-    const int m0 = blockIdx.x * PZ_GATHER_TM, r0 = blockIdx.y * PZ_GATHER_TR;
-    const int nf = p.l_heat ? 4 : 3;
-    constexpr int PER = PZ_GATHER_TM * PZ_GATHER_TR / 256; // elements a thread moves per field
-    cd v[4][PER];
-#pragma unroll
-    for (int f = 0; f < 4; f++) {
-        const cd *src = f == 0 ? p.us : f == 1 ? p.up : f == 2 ? p.om : p.temp;
-#pragma unroll
-        for (int e = 0; e < PER; e++) {
-            const int t = threadIdx.x + e * 256, mm = t / PZ_GATHER_TR, rr = t % PZ_GATHER_TR;
-            v[f][e] = (f < nf && m0 + mm < nm && r0 + rr < N) ? src[(size_t)(m0 + mm) * N + r0 + rr] : mk(0, 0);
-        }
-    }
-#pragma unroll
-    for (int f = 0; f < 4; f++)
-#pragma unroll
-        for (int e = 0; e < PER; e++) {
-            const int t = threadIdx.x + e * 256;
-            tile[f][t / PZ_GATHER_TR][t % PZ_GATHER_TR] = v[f][e];
-        }
-    __syncthreads();
-    for (int f = 0; f < nf; f++) {
-        cd *dst = p.rrow + f * F;
-#pragma unroll
-        for (int e = 0; e < PER; e++) {
-            const int t = threadIdx.x + e * 256, rr = t / PZ_GATHER_TM, mm = t % PZ_GATHER_TM;
-            if (m0 + mm < nm && r0 + rr < N) dst[(size_t)(r0 + rr) * nm + m0 + mm] = tile[f][mm][rr];
-        }
-    }
-}
-
-#define PZ_RADIAL_BIG_THREADS 1024
-__global__ void __launch_bounds__(PZ_RADIAL_BIG_THREADS) k_radial_loop_big(const PzDev *__restrict__ pd, int is, int courant)
-{
-    radial_loop_big_body(*pd, blockIdx.x, is, courant);
-}
-// 512 threads within 128 registers: two workgroups (2 x 67 KB of LDS) share
-// a CU, so the 257 radii of n_r = 257 run in one round on 256 CUs
-#define PZ_RADIAL_INPLACE_THREADS 512
-__global__ void __launch_bounds__(PZ_RADIAL_INPLACE_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
-k_radial_loop_inplace(const PzDev *__restrict__ pd, int is, int courant)
-{
-    radial_loop_inplace_body(*pd, blockIdx.x, is, courant);
-}
-// pz_fft / pz_ifft by the in-place transforms of the long grids, one
-// radius per block (grid real [rad][n_phi], spectral [rad][nm])
-__global__ void __launch_bounds__(PZ_RADIAL_INPLACE_THREADS)
-k_phi_fft_inplace(const PzDev *__restrict__ pd, const double *grid, cd *spec)
-{
-    extern __shared__ double smem[];
-    const PzDev &p = *pd;
-    const int n = p.nphi, nm = p.nm, n2 = (n + 63) >> 6;
-    cd *a = (cd *)smem, *t1 = a + 2 * n, *t2 = t1 + 64, *om = t2 + n2;
-    for (int k = threadIdx.x; k < 64 + n2; k += blockDim.x) t1[k] = p.twid[k < 64 ? k : 64 * (k - 64)];
-    const double *g = grid + (size_t)blockIdx.x * n;
-    for (int j = threadIdx.x; j < n; j += blockDim.x) a[j] = mk(g[j], 0.0);
-    __syncthreads();
-    fft_inplace(a, n, 1, -1, p.radices, p.nrad, [=](int k) { return cmul(t1[k & 63], t2[k >> 6]); }, om);
-    for (int i = threadIdx.x; i < nm; i += blockDim.x) spec[(size_t)blockIdx.x * nm + i] = cdivr(a[i], (double)n);
-}
-__global__ void __launch_bounds__(PZ_RADIAL_INPLACE_THREADS)
-k_phi_ifft_inplace(const PzDev *__restrict__ pd, const cd *spec, double *grid)
-{
-    extern __shared__ double smem[];
-    const PzDev &p = *pd;
-    const int n = p.nphi, nm = p.nm, n2 = (n + 63) >> 6;
-    cd *a = (cd *)smem, *t1 = a + 2 * n, *t2 = t1 + 64, *om = t2 + n2;
-    for (int k = threadIdx.x; k < 64 + n2; k += blockDim.x) t1[k] = p.twid[k < 64 ? k : 64 * (k - 64)];
-    const cd *s = spec + (size_t)blockIdx.x * nm;
-    for (int k = threadIdx.x; k < n; k += blockDim.x) {
-        cd z = mk(0, 0);
-        if (k == 0) z = mk(s[0].x, 0.0);
-        else if (k < nm) z = s[k];
-        else if (n - k < nm) z = cconj(s[n - k]);
-        a[k] = z;
-    }
-    __syncthreads();
-    fft_inplace(a, n, 1, +1, p.radices, p.nrad, [=](int k) {
-        const cd w = cmul(t1[k & 63], t2[k >> 6]);
-        return mk(w.x, -w.y);
-    }, om);
-    for (int j = threadIdx.x; j < n; j += blockDim.x) grid[(size_t)blockIdx.x * n + j] = a[j].x;
-}
-
-__global__ void __launch_bounds__(256) k_radial_loop(const PzDev *__restrict__ pd, int is, int courant)
-{
-    radial_loop_body(*pd, blockIdx.x, is, courant);
-}
-__global__ void __launch_bounds__(256) k_radial_loop_batch(PzBatch b, int is, int courant)
-{
-    const int2 e = b.map[blockIdx.x];
-    radial_loop_body(*b.runs[e.x], e.y, is, courant);
-}
-
-// ---------------------------------------------------------------------------
 // Courant decision and time-scheme weights on the device:
 // dt_courant (courant.f90:78-167), set_dt_array and set_weights
 // (multistep_schemes.f90:137-348; dirk_schemes.f90:275-771), lMat logic of
@@ -1284,14 +786,19 @@ __device__ void scheme_weights(const PzDev &p, PzScheme *s, int *lMatNext)
         if (s->wimp_lin[0] != wimp_old) *lMatNext = 1;
     } else {
         s->wimp_lin[0] = s->dt[0] * p.wimp_lin0;
-        for (int i = 0; i < PZ_MAX_STAGES; i++) {
-            for (int j = 0; j < PZ_MAX_STAGES; j++) {
-                s->bimp[i][j] = s->dt[0] * p.bimp0[i][j];
-                s->bexp[i][j] = s->dt[0] * p.bexp0[i][j];
-            }
-            s->bass_imp[i] = s->dt[0] * p.bass_imp0[i];
-            s->bass_exp[i] = s->dt[0] * p.bass_exp0[i];
-        }
+    }
+}
+// the dt-scaled Butcher tables of a DIRK scheme, one entry per thread
+__device__ __forceinline__ void scheme_tables(const PzDev &p, PzScheme *s, double dt, int t, int nt)
+{
+    if (p.family == 0) return;
+    for (int e = t; e < PZ_MAX_STAGES * PZ_MAX_STAGES; e += nt) {
+        (&s->bimp[0][0])[e] = dt * (&p.bimp0[0][0])[e];
+        (&s->bexp[0][0])[e] = dt * (&p.bexp0[0][0])[e];
+    }
+    for (int e = t; e < PZ_MAX_STAGES; e += nt) {
+        s->bass_imp[e] = dt * p.bass_imp0[e];
+        s->bass_exp[e] = dt * p.bass_exp0[e];
     }
 }
 
@@ -1301,23 +808,14 @@ __global__ void k_set_weights(const PzDev p __attribute__((grid_constant)))
         PzScheme *s = p.ss;
         int dummy = 0;
         scheme_weights(p, s, &dummy);
+        scheme_tables(p, s, s->dt[0], 0, 1);
         // dummy Courant limits before the first radial loop (step_time.f90:124-126)
         for (int i = 0; i < p.N; i++) { p.dtr[i] = 1.0e10; p.dth[i] = 1.0e10; }
     }
 }
 
-__device__ __forceinline__ void courant_body(const PzDev &p)
+__device__ void courant_decide_one(const PzDev &p, PzScheme *s, double dtr, double dth)
 {
-    __shared__ double red[8];
-    PzScheme *s = p.ss;
-    double dtr = 1.0e300, dth = 1.0e300;
-    for (int i = threadIdx.x; i < p.N; i += blockDim.x) {
-        dtr = fmin(dtr, p.dtr[i]);
-        dth = fmin(dth, p.dth[i]);
-    }
-    dtr = -block_reduce(-dtr, red, 1);
-    dth = -block_reduce(-dth, red, 1);
-    if (threadIdx.x != 0) return;
     double dtMax = p.dtMax, dt = s->dt[0];
     double dt_r = fmin(dtr, 1000.0 * dtMax), dt_h = fmin(dth, 1000.0 * dtMax);
     double dt_rh = fmin(dt_r, dt_h);
@@ -1363,6 +861,564 @@ __device__ __forceinline__ void courant_body(const PzDev &p)
     s->n_steps += 1;
 }
 
+// dt_courant, the dt roll and the weights from the smallest Courant limits of
+// the radii; called by every thread of a workgroup with the same limits
+__device__ __forceinline__ void courant_decide(const PzDev &p, double dtr, double dth, double *lds)
+{
+    PzScheme *s = p.ss;
+    if (threadIdx.x == 0) {
+        courant_decide_one(p, s, dtr, dth);
+        lds[0] = s->dt[0];
+    }
+    __syncthreads();
+    scheme_tables(p, s, lds[0], threadIdx.x, blockDim.x);
+}
+// The same decision at the end of a radial loop (courant = 2): every
+// workgroup (one per radius) folds its limits into two minima with device-wide
+// atomics, counts itself, and the one that comes last takes the decision and
+// resets the counters.  The minima are complete when the count is: each
+// workgroup's own atomics have returned before it counts.  Positive doubles
+// compare like their bit patterns, so the limits are those of k_courant.  Saves
+// a launch of one workgroup, 4.5 to 7.3 us of a step.  lds: 8 doubles.
+__device__ __forceinline__ void courant_tail(const PzDev &p, double dtrk, double dthk, double *lds)
+{
+    int *last = (int *)(lds + 4);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long *acc = p.cacc;
+        const unsigned long long big = (unsigned long long)__double_as_longlong(1.0e300);
+        __hip_atomic_fetch_min(acc, (unsigned long long)__double_as_longlong(dtrk), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_fetch_min(acc + 1, (unsigned long long)__double_as_longlong(dthk), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const unsigned long long n = __hip_atomic_fetch_add(acc + 2, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *last = n == (unsigned long long)(p.N - 1);
+        if (*last) {
+            const unsigned long long a = __hip_atomic_exchange(acc, big, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long b = __hip_atomic_exchange(acc + 1, big, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_exchange(acc + 2, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            lds[0] = __longlong_as_double((long long)a);
+            lds[1] = __longlong_as_double((long long)b);
+        }
+    }
+    __syncthreads();
+    if (*last) courant_decide(p, lds[0], lds[1], lds + 2);
+}
+
+// ---------------------------------------------------------------------------
+// Radial loop: rloop::radial_loop (radial_loop.f90:264-392) for one radius
+// per workgroup.  Real fields travel in pairs through one complex FFT.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void radial_loop_body(const PzDev &p, int nr, int is, int courant)
+{
+    extern __shared__ double smem[];
+    const int n = p.nphi, nm = p.nm, N = p.N;
+    const size_t F = (size_t)nm * N;
+    cd *spec = (cd *)smem;           // 5 x nm
+    cd *bufa = spec + 5 * nm;        // 3 x n
+    cd *bufb = bufa + 3 * n;         // 3 x n
+    cd *twl = bufb + 3 * n;          // n twiddles exp(-2 pi i k / n)
+    double *red = (double *)(twl + n);
+    const int nin = (p.l_heat || p.l_chem) ? (p.l_chem ? 3 : 2) : 2;
+
+    for (int k = threadIdx.x; k < n; k += blockDim.x) twl[k] = p.twid[k];
+    for (int i = threadIdx.x; i < nm; i += blockDim.x) {
+        size_t q = (size_t)i * N + nr;
+        spec[i] = p.us[q];
+        spec[nm + i] = p.up[q];
+        spec[2 * nm + i] = p.om[q];
+        spec[3 * nm + i] = p.l_heat ? p.temp[q] : mk(0, 0);
+        spec[4 * nm + i] = p.l_chem ? p.xi[q] : mk(0, 0);
+    }
+    lds_barrier();
+    // Reynolds-stress m-sum (radial_loop.f90:267-278)
+    double part = 0.0;
+    for (int i = threadIdx.x; i < nm; i += blockDim.x) {
+        int m = p.idx2m[i];
+        cd usf = m == 0 ? cscale(0.5 * p.ek * p.CorFac * p.ekpump[nr], spec[nm + i]) : spec[i];
+        part += cc22real(usf, spec[2 * nm + i], m);
+    }
+    double usom = block_reduce(part, red, 0);
+    // pairs (us,up), (om,T), (xi,0) as Hermitian spectra of z = a + i b
+    auto packed = [=](int tr, int k) {
+        // a + i b from the m < n_m half, its conjugate from the other
+        const bool lo = k < nm, hi = !lo && n - k < nm;
+        const int kk = lo ? k : n - k;
+        if (!lo && !hi) return mk(0.0, 0.0);
+        const cd a = spec[(2 * tr) * nm + kk];
+        const cd b = (2 * tr + 1) < 5 ? spec[(2 * tr + 1) * nm + kk] : mk(0.0, 0.0);
+        if (k == 0) return mk(a.x, b.x);
+        return lo ? mk(a.x - b.y, a.y + b.x) : mk(a.x + b.y, b.x - a.y);
+    };
+    // register FFTs (one wave per transform, packing as they load) where
+    // n_phi = 64 P, else LDS Stockham FFTs of the packed columns
+    const int Pw = wave_fft_p_phi(n);
+    cd *g;
+    if (Pw) {
+        fft_wave_phi(Pw, nin, packed, [=](int tr, int k, cd v) { bufb[tr * n + k] = v; },
+                     [=](int k) { const cd w = twl[k]; return mk(w.x, -w.y); });
+        lds_barrier();
+        g = bufb;
+    } else {
+        for (int t = threadIdx.x; t < nin * n; t += blockDim.x) {
+            const int tr = t / n;
+            bufa[t] = packed(tr, t - tr * n);
+        }
+        lds_barrier();
+        g = fft_stockham(bufa, bufb, n, nin, +1, p.radices, p.nrad,
+                         [&](int k) { const cd w = twl[k]; return mk(w.x, -w.y); });
+    }
+    cd *o = (g == bufa) ? bufb : bufa;
+    // Courant (courant.f90:41-76)
+    double dtrk = 1.0e10, dthk = 1.0e10; // thread 0
+    if (courant) {
+        double vr = 0.0, vh = 0.0;
+        for (int j = threadIdx.x; j < n; j += blockDim.x) {
+            cd z = g[j];
+            vr = fmax(vr, z.x * z.x);
+            vh = fmax(vh, z.y * z.y);
+        }
+        vr = block_reduce(vr, red, 1);
+        vh = block_reduce(vh, red, 1);
+        if (threadIdx.x == 0) {
+            double cf = p.courfac;
+            vr = cf * cf * vr;
+            vh = cf * cf * vh;
+            if (vr != 0.0) dtrk = fmin(dtrk, sqrt(p.delxr2[nr] / vr));
+            if (vh != 0.0) dthk = fmin(dthk, sqrt(p.delxh2[nr] / vh));
+            p.dtr[nr] = dtrk;
+            p.dth[nr] = dthk;
+        }
+    }
+    // nonlinear products (radial_loop.f90:316-325): (upX + i r us X)
+    const double rr = p.r[nr];
+    const int nout = 1 + (p.l_heat ? 1 : 0) + (p.l_chem ? 1 : 0); // omega, then T and xi as present
+    for (int j = threadIdx.x; j < n; j += blockDim.x) {
+        cd z0 = g[j], z1 = g[n + j];
+        double us = z0.x, up = z0.y, om = z1.x, T = z1.y;
+        o[j] = mk(up * om, rr * us * om);
+        if (p.l_heat) o[n + j] = mk(up * T, rr * us * T);
+        if (p.l_chem) {
+            double X = g[2 * n + j].x;
+            o[(p.l_heat ? 2 : 1) * n + j] = mk(up * X, rr * us * X);
+        }
+    }
+    lds_barrier();
+    cd *other = (o == bufa) ? bufb : bufa;
+    cd *Z;
+    if (Pw) {
+        fft_wave_phi(Pw, nout, [=](int tr, int i) { return o[tr * n + i]; },
+                     [=](int tr, int k, cd v) { other[tr * n + k] = v; }, [=](int k) { return twl[k]; });
+        lds_barrier();
+        Z = other;
+    } else {
+        Z = fft_stockham(o, other, n, nout, -1, p.radices, p.nrad, [&](int k) { return twl[k]; });
+    }
+    // unpack, normalise and post-scale (radial_loop.f90:350-386)
+    const double or1 = p.or1[nr];
+    const double fbeta = (1.0 - p.tadvz) * p.beta[nr] * or1;
+    for (int t = threadIdx.x; t < nout * nm; t += blockDim.x) {
+        int tr = t / nm, i = t - tr * nm;
+        cd zk = Z[tr * n + i], zc = cconj(Z[tr * n + (i == 0 ? 0 : n - i)]);
+        cd A = mk(0.5 * (zk.x + zc.x), 0.5 * (zk.y + zc.y));  // spectrum of up*X
+        cd B = mk(0.5 * (zk.y - zc.y), -0.5 * (zk.x - zc.x)); // spectrum of r us X
+        A = cdivr(A, (double)n);
+        B = cdivr(B, (double)n);
+        int m = p.idx2m[i];
+        size_t q = (size_t)i * N + nr;
+        cd cim = mk(0.0, -or1 * (double)m); // -or1*ci*m
+        if (tr == 0) {
+            p.P_expl[is * F + q] = (i == 0) ? mk(-usom, 0.0) : cmul(cim, A);
+            p.dVsOm[q] = B;
+        } else if (tr == 1 && p.l_heat) {
+            cd v = cmul(cim, A);
+            p.T_expl[is * F + q] = mk(v.x - fbeta * B.x, v.y - fbeta * B.y);
+            p.dVsT[q] = B;
+        } else {
+            p.X_expl[is * F + q] = cmul(cim, A);
+            p.dVsXi[q] = B;
+        }
+    }
+    if (courant == 2) courant_tail(p, dtrk, dthk, red + 8);
+}
+
+// The radial loop for long azimuthal grids (n_phi too large for the staged
+// variant above): the spectra are packed straight from global memory and
+// the real fields travel through the complex FFTs one pair at a time, so
+// LDS holds four columns of n_phi values (three fields and one scratch).
+__device__ __forceinline__ void radial_loop_big_body(const PzDev &p, int nr, int is, int courant)
+{
+    extern __shared__ double smem[];
+    const int n = p.nphi, nm = p.nm, N = p.N;
+    const size_t F = (size_t)nm * N;
+    cd *s0 = (cd *)smem, *s1 = s0 + n, *s2 = s1 + n, *sc = s2 + n;
+    double *red = (double *)(sc + n);
+    // without composition the third column holds the twiddle table
+    const bool twl_lds = !p.l_chem;
+    cd *twl = s2;
+    if (twl_lds)
+        for (int k = threadIdx.x; k < n; k += blockDim.x) twl[k] = p.twid[k];
+    auto fwd = [&](int k) { return twl_lds ? twl[k] : p.twid[k]; };
+    auto bwd = [&](int k) {
+        const cd w = twl_lds ? twl[k] : p.twid[k];
+        return mk(w.x, -w.y);
+    };
+    // Reynolds-stress m-sum (radial_loop.f90:267-278)
+    double part = 0.0;
+    for (int i = threadIdx.x; i < nm; i += blockDim.x) {
+        const int m = p.idx2m[i];
+        const size_t q = (size_t)i * N + nr;
+        const cd usf = m == 0 ? cscale(0.5 * p.ek * p.CorFac * p.ekpump[nr], p.up[q]) : p.us[q];
+        part += cc22real(usf, p.om[q], m);
+    }
+    const double usom = block_reduce(part, red, 0);
+    // Hermitian spectra of z = a + i b for (us, up), (om, T), (xi, 0)
+    for (int t = threadIdx.x; t < 3 * n; t += blockDim.x) {
+        const int tr = t / n, k = t - tr * n;
+        if (tr == 2 && !p.l_chem) break;
+        const cd *A = tr == 0 ? p.us : (tr == 1 ? p.om : p.xi);
+        const cd *B = tr == 0 ? p.up : (tr == 1 ? (p.l_heat ? p.temp : nullptr) : nullptr);
+        cd z = mk(0, 0);
+        if (k == 0) {
+            z = mk(A[nr].x, B ? B[nr].x : 0.0);
+        } else if (k < nm) {
+            const cd a = A[(size_t)k * N + nr], b = B ? B[(size_t)k * N + nr] : mk(0, 0);
+            z = mk(a.x - b.y, a.y + b.x);
+        } else if (n - k < nm) {
+            const int kk = n - k;
+            const cd a = cconj(A[(size_t)kk * N + nr]), b = B ? cconj(B[(size_t)kk * N + nr]) : mk(0, 0);
+            z = mk(a.x - b.y, a.y + b.x);
+        }
+        (tr == 0 ? s0 : (tr == 1 ? s1 : s2))[k] = z;
+    }
+    lds_barrier();
+    // one complex FFT at a time; the result lands in the column or in the
+    // scratch, whose roles are then exchanged
+    {
+        cd *g = fft_stockham(s0, sc, n, 1, +1, p.radices, p.nrad, bwd);
+        if (g != s0) { sc = s0; s0 = g; }
+        lds_barrier();
+        g = fft_stockham(s1, sc, n, 1, +1, p.radices, p.nrad, bwd);
+        if (g != s1) { sc = s1; s1 = g; }
+        if (p.l_chem) {
+            lds_barrier();
+            g = fft_stockham(s2, sc, n, 1, +1, p.radices, p.nrad, bwd);
+            if (g != s2) { sc = s2; s2 = g; }
+        }
+        lds_barrier();
+    }
+    double dtrk = 1.0e10, dthk = 1.0e10; // thread 0
+    if (courant) {
+        double vr = 0.0, vh = 0.0;
+        for (int j = threadIdx.x; j < n; j += blockDim.x) {
+            const cd z = s0[j];
+            vr = fmax(vr, z.x * z.x);
+            vh = fmax(vh, z.y * z.y);
+        }
+        vr = block_reduce(vr, red, 1);
+        vh = block_reduce(vh, red, 1);
+        if (threadIdx.x == 0) {
+            const double cf = p.courfac;
+            vr = cf * cf * vr;
+            vh = cf * cf * vh;
+            if (vr != 0.0) dtrk = fmin(dtrk, sqrt(p.delxr2[nr] / vr));
+            if (vh != 0.0) dthk = fmin(dthk, sqrt(p.delxh2[nr] / vh));
+            p.dtr[nr] = dtrk;
+            p.dth[nr] = dthk;
+        }
+    }
+    // nonlinear products in place (radial_loop.f90:316-325): (up X + i r us X)
+    const double rr = p.r[nr];
+    for (int j = threadIdx.x; j < n; j += blockDim.x) {
+        const cd z0 = s0[j], z1 = s1[j];
+        const double us = z0.x, up = z0.y, om = z1.x, T = z1.y;
+        const double X = p.l_chem ? s2[j].x : 0.0;
+        s0[j] = mk(up * om, rr * us * om);
+        s1[j] = mk(up * T, rr * us * T);
+        if (p.l_chem) s2[j] = mk(up * X, rr * us * X);
+    }
+    lds_barrier();
+    {
+        cd *g = fft_stockham(s0, sc, n, 1, -1, p.radices, p.nrad, fwd);
+        if (g != s0) { sc = s0; s0 = g; }
+        if (p.l_heat) {
+            lds_barrier();
+            g = fft_stockham(s1, sc, n, 1, -1, p.radices, p.nrad, fwd);
+            if (g != s1) { sc = s1; s1 = g; }
+        }
+        if (p.l_chem) {
+            lds_barrier();
+            g = fft_stockham(s2, sc, n, 1, -1, p.radices, p.nrad, fwd);
+            if (g != s2) { sc = s2; s2 = g; }
+        }
+        lds_barrier();
+    }
+    // unpack, normalise and post-scale (radial_loop.f90:350-386)
+    const double or1 = p.or1[nr];
+    const double fbeta = (1.0 - p.tadvz) * p.beta[nr] * or1;
+    for (int t = threadIdx.x; t < 3 * nm; t += blockDim.x) {
+        const int tr = t / nm, i = t - tr * nm;
+        if ((tr == 1 && !p.l_heat) || (tr == 2 && !p.l_chem)) continue;
+        const cd *Z = tr == 0 ? s0 : (tr == 1 ? s1 : s2);
+        const cd zk = Z[i], zc = cconj(Z[i == 0 ? 0 : n - i]);
+        cd A = mk(0.5 * (zk.x + zc.x), 0.5 * (zk.y + zc.y));
+        cd B = mk(0.5 * (zk.y - zc.y), -0.5 * (zk.x - zc.x));
+        A = cdivr(A, (double)n);
+        B = cdivr(B, (double)n);
+        const int m = p.idx2m[i];
+        const size_t q = (size_t)i * N + nr;
+        const cd cim = mk(0.0, -or1 * (double)m);
+        if (tr == 0) {
+            p.P_expl[is * F + q] = (i == 0) ? mk(-usom, 0.0) : cmul(cim, A);
+            p.dVsOm[q] = B;
+        } else if (tr == 1) {
+            const cd v = cmul(cim, A);
+            p.T_expl[is * F + q] = mk(v.x - fbeta * B.x, v.y - fbeta * B.y);
+            p.dVsT[q] = B;
+        } else {
+            p.X_expl[is * F + q] = cmul(cim, A);
+            p.dVsXi[q] = B;
+        }
+    }
+    if (courant == 2) courant_tail(p, dtrk, dthk, red + 8);
+}
+
+// Long azimuthal grids without composition, where two columns of n_phi and
+// the in-place transforms fit (fft_inplace_fits): the spectra by radius
+// come from k_gather_r (contiguous rows), the pairs (u_s, u_phi) and
+// (omega, T) travel through their in-place complex FFTs together, and LDS
+// holds the two columns and a two-level twiddle table (64 + n_phi / 64
+// entries).
+__device__ __forceinline__ void radial_loop_inplace_body(const PzDev &p, int nr, int is, int courant)
+{
+    extern __shared__ double smem[];
+    const int n = p.nphi, nm = p.nm, N = p.N;
+    const size_t F = (size_t)nm * N;
+    cd *s0 = (cd *)smem, *s1 = s0 + n, *t1 = s1 + n, *t2 = t1 + 64;
+    const int n2 = (n + 63) >> 6;
+    cd *om = t2 + n2;
+    double *red = (double *)(om + PZ_FFT_OM_MAX), *msr = red + 16;
+    const cd *Rus = p.rrow + (size_t)nr * nm, *Rup = Rus + F, *Rom = Rus + 2 * F, *RT = Rus + 3 * F;
+    // exp(-2 pi i k / n) = t1[k mod 64] t2[k / 64]
+    for (int k = threadIdx.x; k < 64 + n2; k += blockDim.x) t1[k] = p.twid[k < 64 ? k : 64 * (k - 64)];
+    auto fwd = [=](int k) { return cmul(t1[k & 63], t2[k >> 6]); };
+    auto bwd = [=](int k) {
+        const cd w = cmul(t1[k & 63], t2[k >> 6]);
+        return mk(w.x, -w.y);
+    };
+    // Hermitian spectra of z = a + i b for (us, up), (om, T), and the
+    // Reynolds-stress m-sum (radial_loop.f90:267-278) from the same loads,
+    // one partial sum per wave in msr (added at the unpack)
+    const double ekc = 0.5 * p.ek * p.CorFac * p.ekpump[nr];
+    double part = 0.0;
+    for (int k = threadIdx.x; k < n; k += blockDim.x) {
+        cd z0 = mk(0, 0), z1 = mk(0, 0);
+        if (k < nm) {
+            const cd us = Rus[k], up = Rup[k], o = Rom[k], T = p.l_heat ? RT[k] : mk(0, 0);
+            const int m = p.idx2m[k];
+            part += cc22real(m == 0 ? cscale(ekc, up) : us, o, m);
+            if (k == 0) {
+                z0 = mk(us.x, up.x);
+                z1 = mk(o.x, T.x);
+            } else {
+                z0 = mk(us.x - up.y, us.y + up.x);
+                z1 = mk(o.x - T.y, o.y + T.x);
+            }
+        } else if (n - k < nm) {
+            const int kk = n - k;
+            const cd us = cconj(Rus[kk]), up = cconj(Rup[kk]), o = cconj(Rom[kk]);
+            const cd T = p.l_heat ? cconj(RT[kk]) : mk(0, 0);
+            z0 = mk(us.x - up.y, us.y + up.x);
+            z1 = mk(o.x - T.y, o.y + T.x);
+        }
+        s0[k] = z0;
+        s1[k] = z1;
+    }
+    for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
+    if ((threadIdx.x & 63) == 0) msr[threadIdx.x >> 6] = part;
+    lds_barrier();
+    fft_inplace(s0, n, 2, +1, p.radices, p.nrad, bwd, om);
+    double dtrk = 1.0e10, dthk = 1.0e10; // thread 0
+    if (courant) {
+        double vr = 0.0, vh = 0.0;
+        for (int j = threadIdx.x; j < n; j += blockDim.x) {
+            const cd z = s0[j];
+            vr = fmax(vr, z.x * z.x);
+            vh = fmax(vh, z.y * z.y);
+        }
+        vr = block_reduce(vr, red, 1);
+        vh = block_reduce(vh, red, 1);
+        if (threadIdx.x == 0) {
+            const double cf = p.courfac;
+            vr = cf * cf * vr;
+            vh = cf * cf * vh;
+            if (vr != 0.0) dtrk = fmin(dtrk, sqrt(p.delxr2[nr] / vr));
+            if (vh != 0.0) dthk = fmin(dthk, sqrt(p.delxh2[nr] / vh));
+            p.dtr[nr] = dtrk;
+            p.dth[nr] = dthk;
+        }
+    }
+    // nonlinear products in place (radial_loop.f90:316-325): (up X + i r us X)
+    const double rr = p.r[nr];
+    for (int j = threadIdx.x; j < n; j += blockDim.x) {
+        const cd z0 = s0[j], z1 = s1[j];
+        const double us = z0.x, up = z0.y, om = z1.x, T = z1.y;
+        s0[j] = mk(up * om, rr * us * om);
+        s1[j] = mk(up * T, rr * us * T);
+    }
+    lds_barrier();
+    fft_inplace(s0, n, p.l_heat ? 2 : 1, -1, p.radices, p.nrad, fwd, om);
+    // unpack, normalise and post-scale (radial_loop.f90:350-386)
+    const double or1 = p.or1[nr];
+    const double fbeta = (1.0 - p.tadvz) * p.beta[nr] * or1;
+    const int nout = p.l_heat ? 2 : 1;
+    for (int t = threadIdx.x; t < nout * nm; t += blockDim.x) {
+        const int tr = t >= nm, i = t - tr * nm;
+        const cd *Z = tr == 0 ? s0 : s1;
+        const cd zk = Z[i], zc = cconj(Z[i == 0 ? 0 : n - i]);
+        cd A = mk(0.5 * (zk.x + zc.x), 0.5 * (zk.y + zc.y));
+        cd B = mk(0.5 * (zk.y - zc.y), -0.5 * (zk.x - zc.x));
+        A = cdivr(A, (double)n);
+        B = cdivr(B, (double)n);
+        const int m = p.idx2m[i];
+        const size_t q = (size_t)i * N + nr;
+        const cd cim = mk(0.0, -or1 * (double)m);
+        if (tr == 0) {
+            if (i == 0) {
+                double usom = msr[0];
+                for (int w = 1; w < (int)((blockDim.x + 63) >> 6); w++) usom += msr[w];
+                p.P_expl[is * F + q] = mk(-usom, 0.0);
+            } else {
+                p.P_expl[is * F + q] = cmul(cim, A);
+            }
+            p.dVsOm[q] = B;
+        } else {
+            const cd v = cmul(cim, A);
+            p.T_expl[is * F + q] = mk(v.x - fbeta * B.x, v.y - fbeta * B.y);
+            p.dVsT[q] = B;
+        }
+    }
+    if (courant == 2) courant_tail(p, dtrk, dthk, red + 8);
+}
+
+// u_s, u_phi, omega (and T) from the mode-major layout [m][n_r] to rows by
+// radius [f][n_r][n_m]: 16 x 32 tiles of all fields through LDS, coalesced
+// on both sides, every load of a thread in flight before the one barrier
+#define PZ_GATHER_TM 16
+#define PZ_GATHER_TR 32
+__global__ void __launch_bounds__(256) k_gather_r(const PzDev *__restrict__ pd)
+{
+    const PzDev &p = *pd;
+    __shared__ cd tile[4][PZ_GATHER_TM][PZ_GATHER_TR + 1];
+    const int N = p.N, nm = p.nm;
+    const size_t F = (size_t)nm * N;
+    const int m0 = blockIdx.x * PZ_GATHER_TM, r0 = blockIdx.y * PZ_GATHER_TR;
+    const int nf = p.l_heat ? 4 : 3;
+    constexpr int PER = PZ_GATHER_TM * PZ_GATHER_TR / 256; // elements a thread moves per field
+    cd v[4][PER];
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+        const cd *src = f == 0 ? p.us : f == 1 ? p.up : f == 2 ? p.om : p.temp;
+#pragma unroll
+        for (int e = 0; e < PER; e++) {
+            const int t = threadIdx.x + e * 256, mm = t / PZ_GATHER_TR, rr = t % PZ_GATHER_TR;
+            v[f][e] = (f < nf && m0 + mm < nm && r0 + rr < N) ? src[(size_t)(m0 + mm) * N + r0 + rr] : mk(0, 0);
+        }
+    }
+#pragma unroll
+    for (int f = 0; f < 4; f++)
+#pragma unroll
+        for (int e = 0; e < PER; e++) {
+            const int t = threadIdx.x + e * 256;
+            tile[f][t / PZ_GATHER_TR][t % PZ_GATHER_TR] = v[f][e];
+        }
+    __syncthreads();
+    for (int f = 0; f < nf; f++) {
+        cd *dst = p.rrow + f * F;
+#pragma unroll
+        for (int e = 0; e < PER; e++) {
+            const int t = threadIdx.x + e * 256, rr = t / PZ_GATHER_TM, mm = t % PZ_GATHER_TM;
+            if (m0 + mm < nm && r0 + rr < N) dst[(size_t)(r0 + rr) * nm + m0 + mm] = tile[f][mm][rr];
+        }
+    }
+}
+
+#define PZ_RADIAL_BIG_THREADS 1024
+__global__ void __launch_bounds__(PZ_RADIAL_BIG_THREADS) k_radial_loop_big(const PzDev *__restrict__ pd, int is, int courant)
+{
+    radial_loop_big_body(*pd, blockIdx.x, is, courant);
+}
+// 512 threads within 128 registers: two workgroups (2 x 67 KB of LDS) share
+// a CU, so the 257 radii of n_r = 257 run in one round on 256 CUs
+#define PZ_RADIAL_INPLACE_THREADS 512
+__global__ void __launch_bounds__(PZ_RADIAL_INPLACE_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
+k_radial_loop_inplace(const PzDev *__restrict__ pd, int is, int courant)
+{
+    radial_loop_inplace_body(*pd, blockIdx.x, is, courant);
+}
+// pz_fft / pz_ifft by the in-place transforms of the long grids, one
+// radius per block (grid real [rad][n_phi], spectral [rad][nm])
+__global__ void __launch_bounds__(PZ_RADIAL_INPLACE_THREADS)
+k_phi_fft_inplace(const PzDev *__restrict__ pd, const double *grid, cd *spec)
+{
+    extern __shared__ double smem[];
+    const PzDev &p = *pd;
+    const int n = p.nphi, nm = p.nm, n2 = (n + 63) >> 6;
+    cd *a = (cd *)smem, *t1 = a + 2 * n, *t2 = t1 + 64, *om = t2 + n2;
+    for (int k = threadIdx.x; k < 64 + n2; k += blockDim.x) t1[k] = p.twid[k < 64 ? k : 64 * (k - 64)];
+    const double *g = grid + (size_t)blockIdx.x * n;
+    for (int j = threadIdx.x; j < n; j += blockDim.x) a[j] = mk(g[j], 0.0);
+    __syncthreads();
+    fft_inplace(a, n, 1, -1, p.radices, p.nrad, [=](int k) { return cmul(t1[k & 63], t2[k >> 6]); }, om);
+    for (int i = threadIdx.x; i < nm; i += blockDim.x) spec[(size_t)blockIdx.x * nm + i] = cdivr(a[i], (double)n);
+}
+__global__ void __launch_bounds__(PZ_RADIAL_INPLACE_THREADS)
+k_phi_ifft_inplace(const PzDev *__restrict__ pd, const cd *spec, double *grid)
+{
+    extern __shared__ double smem[];
+    const PzDev &p = *pd;
+    const int n = p.nphi, nm = p.nm, n2 = (n + 63) >> 6;
+    cd *a = (cd *)smem, *t1 = a + 2 * n, *t2 = t1 + 64, *om = t2 + n2;
+    for (int k = threadIdx.x; k < 64 + n2; k += blockDim.x) t1[k] = p.twid[k < 64 ? k : 64 * (k - 64)];
+    const cd *s = spec + (size_t)blockIdx.x * nm;
+    for (int k = threadIdx.x; k < n; k += blockDim.x) {
+        cd z = mk(0, 0);
+        if (k == 0) z = mk(s[0].x, 0.0);
+        else if (k < nm) z = s[k];
+        else if (n - k < nm) z = cconj(s[n - k]);
+        a[k] = z;
+    }
+    __syncthreads();
+    fft_inplace(a, n, 1, +1, p.radices, p.nrad, [=](int k) {
+        const cd w = cmul(t1[k & 63], t2[k >> 6]);
+        return mk(w.x, -w.y);
+    }, om);
+    for (int j = threadIdx.x; j < n; j += blockDim.x) grid[(size_t)blockIdx.x * n + j] = a[j].x;
+}
+
+__global__ void __launch_bounds__(256) k_radial_loop(const PzDev *__restrict__ pd, int is, int courant)
+{
+    radial_loop_body(*pd, blockIdx.x, is, courant);
+}
+__global__ void __launch_bounds__(256) k_radial_loop_batch(PzBatch b, int is, int courant)
+{
+    const int2 e = b.map[blockIdx.x];
+    radial_loop_body(*b.runs[e.x], e.y, is, courant);
+}
+
+__device__ __forceinline__ void courant_body(const PzDev &p)
+{
+    __shared__ double red[8];
+    double dtr = 1.0e300, dth = 1.0e300;
+    for (int i = threadIdx.x; i < p.N; i += blockDim.x) {
+        dtr = fmin(dtr, p.dtr[i]);
+        dth = fmin(dth, p.dth[i]);
+    }
+    dtr = -block_reduce(-dtr, red, 1);
+    dth = -block_reduce(-dth, red, 1);
+    courant_decide(p, dtr, dth, red);
+}
+// the decision by itself, for the stage-granular boundary and schemes without
+// explicit terms at stage 1
 __global__ void __launch_bounds__(256) k_courant(const PzDev *__restrict__ pd) { courant_body(*pd); }
 __global__ void __launch_bounds__(256) k_courant_batch(PzBatch b) { courant_body(*b.runs[b.map[blockIdx.x].x]); }
 

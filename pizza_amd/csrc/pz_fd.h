@@ -430,18 +430,15 @@ __device__ void fd_implicit(const PzDev &p, const RadView &R, const FdView &S, i
     }
 }
 
-// grid (n_m): get_tMat_Rdist (update_temp_fd.f90:387-483) and its xi twin,
+// get_tMat_Rdist (update_temp_fd.f90:387-483) and its xi twin,
 // get_psimat_Rdist (update_psi_fd.f90:608-770) for m /= 0 and
-// get_uphimat_Rdist (:772-836) for m = 0, each factorised in LDS by one thread
-__device__ __forceinline__ void fd_build_body(const PzDev &p, int mi, int force)
+// get_uphimat_Rdist (:772-836) for m = 0, each factorised by one thread in the
+// caller's LDS blocks mT, mX (3 N doubles) and mP (5 N complex), then written
+// to global memory.  Called by every thread of the workgroup of this m; the
+// factors stay in LDS behind a barrier.
+__device__ __forceinline__ void fd_build_body(const PzDev &p, int mi, double *mT, double *mX, cd *mP)
 {
-    extern __shared__ double smem[];
-    if (!force && p.ss->lMat == 0) return;
     const int N = p.N, m = p.idx2m[mi], tid = threadIdx.x;
-    const FdLayout lay(N);
-    char *lb = (char *)smem;
-    double *mT = (double *)(lb + lay.mT), *mX = (double *)(lb + lay.mX);
-    cd *mP = (cd *)(lb + lay.mP);
     double *mU = (double *)mP;
     const RadView R(p.radc, N);
     const FdView S(p.fdc, N);
@@ -540,11 +537,6 @@ __device__ __forceinline__ void fd_build_body(const PzDev &p, int mi, int force)
     }
 }
 
-__global__ void __launch_bounds__(256) k_fd_build(const PzDev *__restrict__ pd, int force)
-{
-    fd_build_body(*pd, blockIdx.x, force);
-}
-
 // LDS of the m-loop kernel (16-byte blocks): the ghosted columns gT, gX, gP
 // of the right-hand sides (then of the solutions) and the factorised
 // systems of this m; small enough for three workgroups per CU at n_r 257.
@@ -636,10 +628,17 @@ __device__ __forceinline__ void fd_mloop_body(const PzDev &p, int mi, int istage
     const bool hT = p.l_heat, hX = p.l_chem;
     const RadView R(p.radc, N);
     const FdView S(p.fdc, N);
-    if (hT) lds_copy(mT, p.fT + off * 3, sizeof(double) * 3 * N);
-    if (hX) lds_copy(mX, p.fX + off * 3, sizeof(double) * 3 * N);
-    if (m == 0) lds_copy(mP, p.fU, sizeof(double) * 3 * N);
-    else lds_copy(mP, p.fP + off * 5, sizeof(cd) * 5 * N);
+    // the factorised systems of this m: rebuilt here when the matrices changed
+    // (a mode needs no other mode's, so a launch of its own that exits at once
+    // in every other step, 4 us of a 110 us step, is not needed)
+    if (istage == 1 && ss->lMat != 0) {
+        fd_build_body(p, mi, mT, mX, mP);
+    } else {
+        if (hT) lds_copy(mT, p.fT + off * 3, sizeof(double) * 3 * N);
+        if (hX) lds_copy(mX, p.fX + off * 3, sizeof(double) * 3 * N);
+        if (m == 0) lds_copy(mP, p.fU, sizeof(double) * 3 * N);
+        else lds_copy(mP, p.fP + off * 5, sizeof(cd) * 5 * N);
+    }
     const double wcur = imex_weight(p, ss, istage);
     const cd z = mk(0.0, 0.0);
     // explicit terms, right-hand sides with their boundary rows (prepare_*_fd)

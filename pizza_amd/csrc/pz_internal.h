@@ -94,6 +94,9 @@ struct PzDev {
     cd *dVsT, *dVsXi, *dVsOm;
     cd *T_old, *T_impl, *T_expl, *X_old, *X_impl, *X_expl, *P_old, *P_impl, *P_expl;
     double *dtr, *dth; // per-radius Courant limits
+    // their minima (as bit patterns) and the workgroups counted so far, for the
+    // decision at the end of the radial loop
+    unsigned long long *cacc;
 
     // m-independent RHS bands, row-major [n_r][2K+1] in column-offset order
     // (entry K+d is column i+d), already multiplied by rnorm
