@@ -329,13 +329,11 @@ int pz_ifft(pz_handle *h, const double *spec, double *grid, int n_rad);
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * allocation).  d_f, d_df and d_ddf are device arrays complex(8)
  * (n_m, n_r_max) in the layout of pz_get_ddr (m fastest); d_ddf = NULL
- * computes the first derivative only (pz_get_dr).  The layout changes are
- * staged through a static device array of 3 x 262144 complex values that
- * each GPU holds until the process ends, so n_m * n_r_max <= 262144
- * (larger sizes return -2).  Asynchronous on the handle's stream
- * (pz_stream); the caller synchronises before reading d_df.  Every call on
- * one GPU shares that GPU's staging array: calls that overlap on one GPU
- * (handles on different streams) race.
+ * computes the first derivative only (pz_get_dr).  n_m * n_r_max <= 262144
+ * (larger sizes return -2).  Nothing is shared between calls: calls of
+ * different handles may overlap, and d_f may be d_df or d_ddf.  Asynchronous
+ * on the handle's stream (pz_stream); the caller synchronises before reading
+ * d_df.
  */
 int pz_get_ddr_noalloc(pz_handle *h, const double *d_f, double *d_df, double *d_ddf, int n_m,
                        int l_dct_in);

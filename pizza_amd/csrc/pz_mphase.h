@@ -999,6 +999,66 @@ __global__ void __launch_bounds__(256) k_dr_vecs(const PzDev p __attribute__((gr
     }
 }
 
+// get_dr / get_ddr of n_m columns in the reference's layout f(n_m, n_r), m
+// fastest: a workgroup reads its V columns (V n_r values, runs of V), transforms
+// them in LDS as k_dr_vecs does, and writes them back in the same layout, so
+// that f and df may be the same array.  One launch and two passes over memory
+// in place of the layout change, transform and two layout changes of the
+// staged form: 4.3 us a call at n_r 33 with 33 columns (13.6 us), 25.9 us at
+// n_r 193 with 1358 (26.4 us; the long Stockham stages bound it).  More columns a workgroup fill its
+// threads (48 butterflies a stage and column at n_r 193) and lengthen the runs;
+// consecutive tiles share a chiplet, whose L2 then holds their common lines.
+__host__ __device__ inline size_t dr_ref_lds(int N, int V)
+{
+    const size_t L = 2 * (size_t)N - 2;
+    return (4 * (size_t)V * N + 4 * V * L + 4 * V + 16) * sizeof(cd);
+}
+// columns a workgroup: as many as leave two workgroups for every CU's worth of
+// LDS (80 KB each) and the chip's 256 CUs at least one
+inline int dr_ref_vectors(int N, int n_m)
+{
+    for (int V = 4; V > 1; V >>= 1)
+        if (dr_ref_lds(N, V) <= 80 * 1024 && n_m >= 256 * V) return V;
+    return 1;
+}
+__global__ void __launch_bounds__(256) k_dr_ref(const PzDev *__restrict__ pd, const cd *f, cd *df, cd *ddf, int n_m, int l_dct_in, int V)
+{
+    extern __shared__ double smem[];
+    const PzDev &p = *pd;
+    const int N = p.N, tiles = (n_m + V - 1) / V, per = (tiles + 7) >> 3;
+    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (tile >= tiles) return;
+    const int m0 = tile * V, nv = min(V, n_m - m0), sh = V == 4 ? 2 : V - 1; // V is 1, 2 or 4
+    cd *a = (cd *)smem, *c = a + V * N, *d1 = c + V * N, *d2 = d1 + V * N, *buf = d2 + V * N;
+    for (int t = threadIdx.x; t < V * N; t += blockDim.x) {
+        const int k = t >> sh, v = t & (V - 1);
+        lds_store(a, v * N + k, v < nv ? gld(f, (size_t)k * n_m + m0 + v) : mk(0.0, 0.0));
+    }
+    lds_barrier();
+    VecSet<const cd> in, cc;
+    VecSet<cd> co, o1, o2;
+    for (int v = 0; v < V; v++) {
+        in.push(a + v * N);
+        co.push(c + v * N);
+        cc.push(l_dct_in ? c + v * N : a + v * N);
+        o1.push(d1 + v * N);
+        if (ddf) o2.push(d2 + v * N);
+    }
+    if (l_dct_in) {
+        dct_fft(p, in, co, V, 0, p.cosT, p.sinT, buf);
+        lds_barrier();
+    }
+    dr_fft(p, RadView(p.radc, N), cc, o1, o2, V, p.cosT, p.sinT, buf);
+    lds_barrier();
+    for (int t = threadIdx.x; t < V * N; t += blockDim.x) {
+        const int k = t >> sh, v = t & (V - 1);
+        if (v >= nv) continue;
+        const size_t q = (size_t)k * n_m + m0 + v;
+        df[q] = lds_load(d1, v * N + k);
+        if (ddf) ddf[q] = lds_load(d2, v * N + k);
+    }
+}
+
 // azimuthal transforms, one radius per block: grid real [rad][n_phi],
 // spectral [rad][nm]
 __global__ void __launch_bounds__(256) k_phi_fft(const PzDev p __attribute__((grid_constant)), const double *grid, cd *spec)
