@@ -428,11 +428,21 @@ __device__ __forceinline__ void coll_uphi0_impl(const PzDev &p, const RadView &R
 // exp_calc, update_temp_co / update_xi_co (update_temp_coll.f90:66-150) and
 // update_om_coll_smat (update_psi_coll_smat.f90:88-321) with their implicit
 // terms (get_*_rhs_imp_coll*).
-template <bool RADLDS>
+//
+// Bound by the chain of phases of one workgroup per mode, so every input
+// (tables, slots, fields, wall values) is loaded before the first is stored,
+// the slots of a multistep scheme rotate from the values read, the barriers
+// order LDS only, and a single run has the first PFS and PFP columns of its
+// inverses in registers long before their products (0: none, for batches,
+// whose workgroups share a CU within 128 registers; the sums are the same).
+// Measured a launch: 48.3 us at n_r 129 and 171 modes (51.8 with loads where
+// they were used), 35.1 us a stage of ARS222 at n_r 49 and 49 modes (37.4),
+// 20.8 us at n_r 33 and 33 modes (23.1).
+template <bool RADLDS, int PFS, int PFP>
 __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, int exp_calc)
 {
     extern __shared__ double smem[];
-    const int N = p.N, m = p.idx2m[mi];
+    const int N = p.N, m = mi * p.minc;
     const size_t F = (size_t)p.nm * N, off = (size_t)mi * N;
     const int is = istage - 1;
     const PzScheme *ss = p.ss;
@@ -453,42 +463,59 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
     // transform tables and radial rows: LDS copies, or global (L2) reads
     const double *cosT = p.cosT, *sinT = p.sinT;
     if (RADLDS) {
-        double *c = (double *)(lb + lay.cosT), *s = (double *)(lb + lay.sinT);
-        lds_copy(c, p.cosT, sizeof(double) * p.L);
-        lds_copy(s, p.sinT, sizeof(double) * p.L);
-        cosT = c;
-        sinT = s;
-        lds_copy(lb + lay.rad, p.radc, sizeof(double) * PZ_NRADC * N);
+        cosT = (const double *)(lb + lay.cosT);
+        sinT = (const double *)(lb + lay.sinT);
     }
     const RadView R(RADLDS ? (const double *)(lb + lay.rad) : p.radc, N);
 
     // ---------------- global inputs -------------------------------------
-    // three groups of N threads: T, xi, psi (three times as many loads in
-    // flight)
+    // three groups of N threads: T, xi, psi
+    const int ntab = 2 * p.L + PZ_NRADC * N;
+    TableStage tab;
+    if (RADLDS) tab.load(p.cosT, ntab);
     for (int t = tid; t < 3 * N; t += blockDim.x) {
         const int g = t / N, k = t - g * N;
-        if (g == 0) {
-            if (hT) eT[k] = p.T_expl[is * F + off + k];
-            Tv[k] = hT ? p.temp[off + k] : mk(0, 0);
-            if (exp_calc && hT) aT[k] = p.dVsT[off + k];
-            if (hT) imex_split(p, ss, istage, p.T_old, p.T_impl, p.T_expl, off, k, PT[k], QT[k]);
-        } else if (g == 1) {
-            if (hX) eX[k] = p.X_expl[is * F + off + k];
-            Xv[k] = hX ? p.xi[off + k] : mk(0, 0);
-            if (exp_calc && hX) aX[k] = p.dVsXi[off + k];
-            if (hX) imex_split(p, ss, istage, p.X_old, p.X_impl, p.X_expl, off, k, PX[k], QX[k]);
-        } else {
-            eP[k] = p.P_expl[is * F + off + k];
-            usv[k] = p.us[off + k];
-            if (exp_calc) aP[k] = p.dVsOm[off + k];
-            if (exp_calc && p.dmat && p.l_ek_pump) {
-                omv[k] = p.om[off + k];
-                upv[k] = p.up[off + k];
-            }
-            imex_split(p, ss, istage, p.P_old, p.P_impl, p.P_expl, off, k, PP[k], QP[k]);
+        const size_t q = off + k, qe = is * F + q;
+        const bool have = g == 0 ? hT : g == 1 ? hX : true, wall = g < 2 && (k == 0 || k == N - 1);
+        cd *old = g == 0 ? p.T_old : g == 1 ? p.X_old : p.P_old, *impl = g == 0 ? p.T_impl : g == 1 ? p.X_impl : p.P_impl;
+        cd *expl = g == 0 ? p.T_expl : g == 1 ? p.X_expl : p.P_expl;
+        const cd *dV = g == 0 ? p.dVsT : g == 1 ? p.dVsXi : p.dVsOm;
+        cd e = mk(0.0, 0.0), a = e, u = e, u2 = e, u3 = e, wv0 = e, b, c;
+        ImexSlots sl;
+        if (have) {
+            e = gld(expl, qe);
+            u = gld(g == 0 ? p.temp : g == 1 ? p.xi : p.us, q);
+            if (exp_calc) a = gld(dV, q);
+            sl.load(p, istage, old, impl, expl, q);
+        }
+        if (wall) wv0 = gld(g == 0 ? (k == 0 ? p.topt : p.bott) : (k == 0 ? p.topxi : p.botxi), mi);
+        if (g == 2 && exp_calc && p.dmat && p.l_ek_pump) {
+            u2 = gld(p.om, q);
+            u3 = gld(p.up, q);
+        }
+        if (RADLDS && t == tid) tab.store(p.cosT, (double *)(lb + lay.cosT), ntab);
+        lds_store(g == 0 ? Tv : g == 1 ? Xv : usv, k, u);
+        if (have) {
+            lds_store(g == 0 ? eT : g == 1 ? eX : eP, k, e);
+            lds_store(g == 0 ? aT : g == 1 ? aX : aP, k, a);
+            sl.sum(p, ss, istage, old, impl, expl, q, b, c);
+            if (wall) b = wv0; // boundary row: the wall value alone
+            lds_store(g == 0 ? PT : g == 1 ? PX : PP, k, b);
+            lds_store(g == 0 ? QT : g == 1 ? QX : QP, k, c);
+        }
+        if (g == 2 && p.dmat) {
+            lds_store(omv, k, u2);
+            lds_store(upv, k, u3);
         }
     }
+    if (RADLDS && tid >= 3 * N) tab.store(p.cosT, (double *)(lb + lay.cosT), ntab);
     const double wcur = imex_weight(p, ss, istage);
+    const VecSet<const double> invS(hT ? p.T_inv + off * ldi : p.X_inv + off * ldi);
+    const VecSet<const cd> invP(p.PC_inv + off * 2 * N);
+    MatAhead<double, 1, PFS ? PFS : 1> preS; // T or xi alone
+    MatAhead<cd, 1, PFP ? PFP : 1> preP;
+    if constexpr (PFS > 0)
+        if (hT != hX) preS.load(N, N, ldi, invS);
     // the groups above wrote vectors that other threads read next, with or
     // without the explicit part
     lds_barrier();
@@ -546,28 +573,33 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
 
     // ---------------- T and xi -------------------------------------------
     for (int k = tid; k < N; k += blockDim.x) {
+        const bool wall = k == 0 || k == N - 1;
         if (hT) {
-            cd r = cadd(cadd(PT[k], cscale(wcur, eT[k])), QT[k]);
-            if (k == 0) r = p.topt[mi];
-            if (k == N - 1) r = p.bott[mi];
-            aT[k] = r;
+            rotate_current(p, p.T_expl, off, k, eT[k]);
+            aT[k] = wall ? PT[k] : cadd(cadd(PT[k], cscale(wcur, eT[k])), QT[k]);
         }
         if (hX) {
-            cd r = cadd(cadd(PX[k], cscale(wcur, eX[k])), QX[k]);
-            if (k == 0) r = p.topxi[mi];
-            if (k == N - 1) r = p.botxi[mi];
-            aX[k] = r;
+            rotate_current(p, p.X_expl, off, k, eX[k]);
+            aX[k] = wall ? PX[k] : cadd(cadd(PX[k], cscale(wcur, eX[k])), QX[k]);
         }
+        rotate_current(p, p.P_expl, off, k, eP[k]);
     }
     lds_barrier();
+    if constexpr (PFP > 0)
+        if (m != 0 && !p.dmat) preP.load(2 * N, N, 2 * N, invP);
     if (hT && hX) {
         const VecSet<const double> inv(p.T_inv + off * ldi, p.X_inv + off * ldi);
         const VecSet<cd> xs(aT, aX);
         block_matvec<double, 2>(N, ldi, inv, xs, xs, red);
     } else if (hT || hX) {
-        const VecSet<const double> inv(hT ? p.T_inv + off * ldi : p.X_inv + off * ldi);
-        const VecSet<cd> xs(hT ? aT : aX);
-        block_matvec<double, 1>(N, ldi, inv, xs, xs, red);
+        cd *x = hT ? aT : aX;
+        if constexpr (PFS > 0) {
+            preS.apply(N, N, ldi, invS, VecSet<cd>(x), red, []() {},
+                       [&](int k, const cd(&s)[1]) __attribute__((always_inline)) { x[k] = s[0]; });
+            lds_barrier();
+        } else {
+            block_matvec<double, 1>(N, ldi, invS, VecSet<cd>(x), VecSet<cd>(x), red);
+        }
     }
     for (int k = nc + tid; k < N; k += blockDim.x) { aT[k] = mk(0, 0); aX[k] = mk(0, 0); }
     lds_barrier();
@@ -593,9 +625,6 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
         if (din.n) dct_fft(p, din, dout, din.n, 0, cosT, sinT, fbuf);
         lds_barrier();
     }
-    if (hT) rotate_row(p, p.T_old, p.T_impl, p.T_expl, off);
-    if (hX) rotate_row(p, p.X_old, p.X_impl, p.X_expl, off);
-    lds_barrier();
     for (int k = tid; k < N; k += blockDim.x) {
         const double o1 = R.or1(k), o2 = R.or2(k);
         if (hT) {
@@ -631,12 +660,8 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
         for (int k = nc + tid; k < N; k += blockDim.x) wv[k] = mk(0, 0);
         lds_barrier();
         // om0 = get_dr(uphi0, l_dct = .false.) (dcheb recursion), uphi0 -> grid
-        double *f = (double *)b2, *df = f + N;
-        for (int k = tid; k < N; k += blockDim.x) f[k] = wv[k].x;
-        lds_barrier();
-        if (tid == 0) dcheb_real(p, f, df);
-        lds_barrier();
-        for (int k = tid; k < N; k += blockDim.x) { cP[k] = mk(df[k], 0.0); eP[k] = mk(f[k], 0.0); }
+        if (tid < 128) dcheb_waves(p, wv, cP);
+        for (int k = tid; k < N; k += blockDim.x) eP[k] = mk(wv[k].x, 0.0);
         lds_barrier();
         {
             const VecSet<const cd> din(cP, eP);
@@ -654,7 +679,6 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
             p.om[off + k] = om;
             p.psi[off + k] = mk(0, 0);
         }
-        rotate_row(p, p.P_old, p.P_impl, p.P_expl, off);
         lds_barrier();
         if (inext == 1)
             for (int k = tid; k < N; k += blockDim.x) p.P_old[off + k] = upv[k];
@@ -712,8 +736,13 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
         lds_barrier();
     } else {
         // [omega; psi] coefficients (2N values in aP, cP)
-        block_matvec_rc<cd, 1>(2 * N, N, 2 * N, VecSet<const cd>(p.PC_inv + off * 2 * N), VecSet<cd>(aP),
-                               VecSet<cd>(aP), red);
+        if constexpr (PFP > 0) {
+            preP.apply(2 * N, N, 2 * N, invP, VecSet<cd>(aP), red, []() {},
+                       [&](int k, const cd(&s)[1]) __attribute__((always_inline)) { aP[k] = s[0]; });
+            lds_barrier();
+        } else {
+            block_matvec_rc<cd, 1>(2 * N, N, 2 * N, invP, VecSet<cd>(aP), VecSet<cd>(aP), red);
+        }
         for (int k = nc + tid; k < N; k += blockDim.x) { aP[k] = mk(0, 0); cP[k] = mk(0, 0); }
         lds_barrier();
     }
@@ -735,8 +764,6 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
         p.up[off + k] = up;
         p.om[off + k] = omv[k];
     }
-    rotate_row(p, p.P_old, p.P_impl, p.P_expl, off);
-    lds_barrier();
     for (int k = tid; k < N; k += blockDim.x) {
         if (inext == 1) p.P_old[off + k] = omv[k];
         if (lcalc) {
@@ -761,20 +788,20 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
 
 __global__ void __launch_bounds__(PZ_MPHASE_THREADS) k_mcoll(const PzDev *__restrict__ pd, int istage, int exp_calc)
 {
-    mcoll_body<true>(*pd, blockIdx.x, istage, exp_calc);
+    mcoll_body<true, 12, 16>(*pd, blockIdx.x, istage, exp_calc);
 }
 // the same with the radial rows and transform tables read through L2, for
 // grids whose full LDS layout does not fit a workgroup (n_r > 193)
 __global__ void __launch_bounds__(PZ_MPHASE_THREADS) k_mcoll_l2(const PzDev *__restrict__ pd, int istage, int exp_calc)
 {
-    mcoll_body<false>(*pd, blockIdx.x, istage, exp_calc);
+    mcoll_body<false, 12, 16>(*pd, blockIdx.x, istage, exp_calc);
 }
 // batched; RADLDS picks the radial rows' place per size class
 template <bool RADLDS>
 __global__ void __launch_bounds__(PZ_MPHASE_THREADS) k_mcoll_batch(PzBatch b, int istage, int exp_calc)
 {
     const int2 e = b.map[blockIdx.x];
-    mcoll_body<RADLDS>(*b.runs[e.x], e.y, istage, exp_calc);
+    mcoll_body<RADLDS, 0, 0>(*b.runs[e.x], e.y, istage, exp_calc);
 }
 
 // get_start_fields, collocation branch (init_fields.f90:191-244): dT/dr,

@@ -40,18 +40,6 @@ __device__ __forceinline__ double imex_weight(const PzDev &p, const PzScheme *s,
     return p.family == 0 ? s->wexp[istage - 1] : s->bexp[istage][istage - 1];
 }
 
-// rotate_imex for one m row (multistep_schemes.f90:462-498); DIRK: no-op
-__device__ __forceinline__ void rotate_row(const PzDev &p, cd *old, cd *impl, cd *expl, size_t off)
-{
-    if (p.family != 0) return;
-    const size_t F = (size_t)p.nm * p.N;
-    for (int k = threadIdx.x; k < p.N; k += blockDim.x) {
-        for (int o = p.nexp - 1; o >= 1; o--) expl[o * F + off + k] = expl[(o - 1) * F + off + k];
-        for (int o = p.nold - 1; o >= 1; o--) old[o * F + off + k] = old[(o - 1) * F + off + k];
-        for (int o = p.nimp - 1; o >= 1; o--) impl[o * F + off + k] = impl[(o - 1) * F + off + k];
-    }
-}
-
 // -BuoFac rgrav/r i m T - ChemFac rgrav/r i m X (update_psi_integ_smat.f90:286-304)
 __device__ __forceinline__ cd buoyancy(const PzDev &p, const RadView &R, int m, int k, cd T, cd X)
 {
