@@ -1860,8 +1860,9 @@ extern "C" int pz_start(pz_handle *h)
         }
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(h->stream));
-        if (h->gexec) { (void)hipGraphExecDestroy(h->gexec); h->gexec = nullptr; }
-        if (h->graph) { (void)hipGraphDestroy(h->graph); h->graph = nullptr; }
+        // the captured step stays: its kernels read everything a start or a
+        // restart changes (fields, slots, scheme state, l_bridge) through the
+        // descriptor and the state block, whose addresses do not change
         h->started = true;
         h->restarted = rst;
         h->rst.pending = false;
