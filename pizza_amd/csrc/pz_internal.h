@@ -15,7 +15,7 @@ typedef double2 cd;
 #define PZ_MAX_STAGES 8
 
 // Time-scheme state that changes during the run.  It lives in device memory
-// and is updated by k_courant, so a captured step replays without the host.
+// and is updated by the Courant decision on the device, so a captured step replays without the host.
 struct PzScheme {
     double dt[8];
     double wimp[8];
