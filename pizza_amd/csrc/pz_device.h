@@ -2366,7 +2366,7 @@ struct TableStage {
 // complex values of scratch for nmat matrices of nrow x ncol with `threads`
 // threads, rpt rows per thread: (CG - 1) partial sums of R row units each
 // (at most 2 threads nmat)
-__host__ __device__ inline size_t matvec_scratch(int nrow, int ncol, int threads, int rpt, int nmat)
+__host__ __device__ constexpr size_t matvec_scratch(int nrow, int ncol, int threads, int rpt, int nmat)
 {
     const int R = (nrow + rpt - 1) / rpt;
     const int CG = threads / R < ncol ? threads / R : ncol;
@@ -2533,7 +2533,7 @@ struct MatAhead {
     }
 };
 // complex values of red for that product
-__host__ __device__ inline size_t ahead_scratch(int nrow, int ncol, int threads, int rpt, int nmat)
+__host__ __device__ constexpr size_t ahead_scratch(int nrow, int ncol, int threads, int rpt, int nmat)
 {
     const int R = (nrow + rpt - 1) / rpt, CG = threads / R < ncol ? threads / R : ncol;
     return (size_t)nmat * CG * R * rpt;

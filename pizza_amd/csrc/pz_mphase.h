@@ -93,11 +93,11 @@ __device__ __forceinline__ void dcheb_real(const PzDev &p, const double *__restr
 // threads of the m-loop kernels for n_r: 256 leave room for more
 // workgroups per CU on small grids (the coupled collocation system needs
 // 2 n_r <= threads)
-__host__ __device__ inline int mloop_threads(int N) { return N <= 65 ? 256 : PZ_MPHASE_THREADS; }
+__host__ __device__ constexpr int mloop_threads(int N) { return N <= 65 ? 256 : PZ_MPHASE_THREADS; }
 
 // column groups of a product with `threads` threads: the partial sums of three
 // vectors must fit the kernel's reduction scratch
-__host__ __device__ inline int shared_groups(int N, int threads)
+__host__ __device__ constexpr int shared_groups(int N, int threads)
 {
     const int rq = (N + 3) / 4, cap = N <= 160 ? 8 : 3;
     int cg = threads / rq;
@@ -105,14 +105,38 @@ __host__ __device__ inline int shared_groups(int N, int threads)
     return cg < N ? cg : N;
 }
 
+// complex values of an m-loop kernel's scratch `red`: the FFT buffers of the
+// Chebyshev transforms (6 L + 12), shared with the partial sums of the dense
+// products.  Each product a kernel may run is listed with the rows, columns
+// and rows a thread it is called with: block_matvec keeps the sums of all
+// column groups but the first in registers (matvec_scratch), MatAhead stores
+// those of every group (ahead_scratch), SharedMv [vector][group][n_r rounded
+// up to 4], with half the threads for T and xi and half for psi.
+__host__ __device__ constexpr size_t mloop_scratch(int N, int threads, bool integ)
+{
+    const size_t ldm = (N + 3) & ~3;
+    const size_t need[] = {6 * (2 * (size_t)N - 2) + 16,
+                           matvec_scratch(N, N, threads, 2, 2),     // T and xi
+                           matvec_scratch(N, N, threads, 1, 1),
+                           matvec_scratch(2 * N, N, threads, 1, 1), // omega and psi
+                           // T, xi: one ahead (collocation), both (integration)
+                           ahead_scratch(N, N, threads, 2, integ ? 2 : 1),
+                           ahead_scratch(integ ? N : 2 * N, N, threads, 1, 1),
+                           integ ? 3 * shared_groups(N, threads / 2) * ldm : 0,
+                           integ ? shared_groups(N, threads) * ldm : 0};
+    size_t most = 0;
+    for (size_t n : need) most = n > most ? n : most;
+    return most;
+}
+
 // LDS layout of k_mphase: working vectors, transform tables and the
 // reduction scratch of the dense solves (16-byte aligned blocks).
 struct MpLayout {
-    size_t vec, cosT, sinT, rad, red, total;
+    size_t vec = 0, cosT = 0, sinT = 0, rad = 0, red = 0, total = 0;
     // rad_lds = false: the radial rows and the transform tables stay in
     // global memory (read through L2), which frees PZ_NRADC n_r + 2 L
     // doubles of LDS per workgroup (collocation m-loop only)
-    __host__ __device__ __forceinline__ MpLayout(int N, int threads, bool rad_lds = true, bool integ = false)
+    __host__ __device__ constexpr MpLayout(int N, int threads, bool rad_lds = true, bool integ = false)
     {
         size_t o = 0;
         auto take = [&](size_t bytes) { size_t r = o; o += (bytes + 15) & ~(size_t)15; return r; };
@@ -122,22 +146,7 @@ struct MpLayout {
         cosT = rad_lds ? take(sizeof(double) * (2 * L + PZ_NRADC * N)) : 0;
         sinT = cosT + sizeof(double) * L;
         rad = cosT + sizeof(double) * 2 * L;
-        // FFT scratch of the Chebyshev transforms (6 L + 12), shared with the
-        // reduction scratch of the dense solves: T and xi together (real),
-        // psi (complex, n_r rows on the integration method, 2 n_r on the
-        // collocation method)
-        size_t mv = matvec_scratch(N, N, threads, 2, 2);
-        const size_t m1 = matvec_scratch(N, N, threads, 1, 1), m2 = matvec_scratch(2 * N, N, threads, 1, 1);
-        if (m1 > mv) mv = m1;
-        if (m2 > mv) mv = m2;
-        // integration method: three vectors' partial sums of the products
-        // with shared matrices, those of the inverses loaded ahead
-        const size_t ldm = (N + 3) & ~3;
-        const size_t need[] = {3 * shared_groups(N, threads / 2) * ldm, shared_groups(N, threads) * ldm,
-                               ahead_scratch(N, N, threads, 2, 2), ahead_scratch(N, N, threads, 1, 1)};
-        for (size_t m3 : need)
-            if (integ && m3 > mv) mv = m3;
-        red = take(sizeof(cd) * ((size_t)(6 * L + 16) > mv ? (size_t)(6 * L + 16) : mv));
+        red = take(sizeof(cd) * mloop_scratch(N, threads, integ));
         total = o;
     }
 };
