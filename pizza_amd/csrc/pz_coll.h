@@ -254,7 +254,7 @@ __device__ __forceinline__ void build_coll_body(const PzDev &p, int mi, int fld,
         cd *W = (cd *)(ws + 2 * regT);
         const int n = 2 * N;
         coll_assemble<cd>(p, R, fld, m, p.hdifV[mi], W, facs, red);
-        const int info = gj_invert<cd>(W, n, N, lds);
+        const int info = gj_invert<cd>(W, n, N, lds, gj_first_psi(N));
         if (tid == 0) p.info[fld * p.nm + mi] = info;
         if (info) return;
         // INV = diag(fac_col) A_s^{-1} diag(fac_row); only the first N

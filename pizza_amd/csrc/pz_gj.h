@@ -105,6 +105,20 @@ __device__ __forceinline__ void gj_tile(const cd *U, int np, const cd *Wk, int c
     for (int r = 0; r < 4; r++) w[r] = mk(re[r], im[r]);
 }
 
+// The first panel of the omega-psi system.  Its omega block has N columns and
+// only N - 2 omega equations (two of its rows are wall conditions on psi), so
+// the pivots N - 2 and N - 1 (counted from 0) come from the rows of omega =
+// -Laplacian(psi), whose omega entries the row scaling leaves at 1e-6.  A group
+// of pivot columns that ends between the two has coefficients U of 1e6, and the
+// columns behind it, formed as U W[K], lose that factor where the
+// column-by-column elimination does not: at n_r 9 the residual of a solve was
+// up to 128 times that of an elimination without panels, 7 times at n_r 17,
+// within the spread of 4 at other n_r.  Groups of 8 end there when N - 1 is a
+// multiple of 8; four columns first put both pivots inside a group (2.1 and
+// 2.7 times).  2 N is then 2 more than a multiple of 16, so the number of panels
+// stays the same.
+__host__ __device__ constexpr int gj_first_psi(int N) { return (N - 1) % 8 == 0 ? 4 : GJ_B; }
+
 // In-place blocked Gauss-Jordan inversion with partial pivoting of the
 // row-major n x n block W by one workgroup of 1024 threads, forming only the
 // columns of A^{-1} that multiply the first nr entries of a right-hand side.
@@ -131,10 +145,11 @@ __device__ __forceinline__ void gj_tile(const cd *U, int np, const cd *Wk, int c
 // Measured, k_build_coll at n_r 129 and 171 modes: 2.1 ms (5.0 ms with the
 // panels and the rank-16 update on the vector unit in LDS, rows swapped); at
 // n_r 49 and 49 modes 0.24 ms (0.65 ms).
+// first: columns of the first panel, 1 .. GJ_B (gj_first_psi).
 // lds: gj_lds_bytes<M>(n).  Returns the LAPACK-style info (k + 1 of the first
 // zero pivot, 0 if none).
 template <class M>
-__device__ int gj_invert(M *W, int n, int nr, char *lds)
+__device__ int gj_invert(M *W, int n, int nr, char *lds, int first = GJ_B)
 {
     constexpr int SB = gj_sub<M>();
     const GjLayout<M> lay(n);
@@ -149,8 +164,8 @@ __device__ int gj_invert(M *W, int n, int nr, char *lds)
     int ndone = 0;     // finished columns that are wanted (slots in done)
     if (tid < 2 * GJ_ROWW) key[tid] = 0.0;
     __syncthreads();
-    for (int k0 = 0; k0 < n; k0 += GJ_B) {
-        const int b = min(GJ_B, n - k0);
+    for (int k0 = 0, b; k0 < n; k0 += b) {
+        b = min(k0 == 0 ? first : GJ_B, n - k0);
         bool inpanel = false; // this thread's row is a pivot row of the panel
         for (int s0 = 0; s0 < b; s0 += SB) {
             const int k1 = k0 + s0, bs = min(SB, b - s0);

@@ -1,6 +1,6 @@
 """The collocation method's m-loop at the sizes and options where its loads
 ahead, its thread groups and its tables take another form: fewer rows than
-columns loaded ahead (8, 10 to 13 and 16, 17), one and several rows a thread,
+columns loaded ahead (8 to 13 and 16, 17), one and several rows a thread,
 register and Stockham FFTs, tables in LDS and in L2 (n_r 97 and 256); T alone,
 xi alone and both; every slot of SBDF4 and the stage sums of ARS443; the
 coupled and the influence-matrix solve.  One and six steps against the oracle, each
@@ -19,6 +19,8 @@ pytestmark = pytest.mark.gpu
 
 CASES = [  # n_r, scheme, ra, raxi, buoyancy, pumping, solve
     (8, "CNAB2", 1e5, 1e5, "IMP", True, "direct"),
+    (9, "SBDF2", 1e5, 0.0, "IMP", True, "direct"),
+    (9, "CNAB2", 1e5, 1e5, "EXP", True, "direct"),
     (10, "SBDF2", 1e5, 0.0, "IMP", True, "direct"),
     (11, "SBDF3", 1e5, 0.0, "IMP", True, "direct"),
     (12, "SBDF4", 1e5, 0.0, "IMP", False, "direct"),
