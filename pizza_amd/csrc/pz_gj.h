@@ -112,12 +112,14 @@ __device__ __forceinline__ void gj_tile(const cd *U, int np, const cd *Wk, int c
 // of pivot columns that ends between the two has coefficients U of 1e6, and the
 // columns behind it, formed as U W[K], lose that factor where the
 // column-by-column elimination does not: at n_r 9 the residual of a solve was
-// up to 128 times that of an elimination without panels, 7 times at n_r 17,
-// within the spread of 4 at other n_r.  Groups of 8 end there when N - 1 is a
-// multiple of 8; four columns first put both pivots inside a group (2.1 and
-// 2.7 times).  2 N is then 2 more than a multiple of 16, so the number of panels
-// stays the same.
-__host__ __device__ constexpr int gj_first_psi(int N) { return (N - 1) % 8 == 0 ? 4 : GJ_B; }
+// up to 128 times that of an elimination without panels, at n_r 17 7 times.
+// Groups of 8 end there when N - 1 is a multiple of 8; four columns first put
+// both pivots inside a group (2.1 and 2.7 times).  From n_r 25 on the loss is
+// lost in the spread between orders of elimination (up to 5 times with either
+// panel, and 20 times at n_r 145 with four columns first in one of eight runs),
+// so the whole panel stays.  2 N is 2 more than a multiple of 16 there: the
+// number of panels is the same.
+__host__ __device__ constexpr int gj_first_psi(int N) { return N <= 17 && (N - 1) % 8 == 0 ? 4 : GJ_B; }
 
 // In-place blocked Gauss-Jordan inversion with partial pivoting of the
 // row-major n x n block W by one workgroup of 1024 threads, forming only the
