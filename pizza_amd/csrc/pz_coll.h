@@ -389,7 +389,7 @@ __device__ __forceinline__ void ddcheb_real(const PzDev &p, const double *__rest
 
 // m = 0 implicit term of get_psi_rhs_imp_coll_smat (update_psi_coll_smat.f90:
 // 454-466): u0 holds u_phi(m = 0) on the grid (real parts); writes impl.
-// Uses cA, cB (LDS vectors) and dt3 (3 N doubles) as scratch.
+// Uses cA, cB (LDS vectors), dt3 (3 N doubles) and fbuf (4 L complex) as scratch.
 __device__ __forceinline__ void coll_uphi0_impl(const PzDev &p, const RadView &R, const cd *u0, cd *cA, cd *cB, double *dt3,
                                 const double *cosT, const double *sinT, cd *fbuf, cd *impl_out, double hdif)
 {
@@ -408,15 +408,18 @@ __device__ __forceinline__ void coll_uphi0_impl(const PzDev &p, const RadView &R
     lds_barrier();
     for (int k = tid; k < N; k += blockDim.x) { cA[k] = mk(df[k], 0.0); cB[k] = mk(ddf[k], 0.0); }
     lds_barrier();
+    // back to the grid: the FFTs work in place, the direct sums of the lengths
+    // without a plan read every input for each output and leave fbuf free
+    cd *gA = p.nradL ? cA : fbuf, *gB = p.nradL ? cB : fbuf + N;
     {
         const VecSet<const cd> din(cA, cB);
-        VecSet<cd> dout(cA, cB);
+        VecSet<cd> dout(gA, gB);
         dct_fft(p, din, dout, 2, 0, cosT, sinT, fbuf);
     }
     lds_barrier();
     for (int k = tid; k < N; k += blockDim.x) {
         const double a = R.drx(k), b = R.ddrx(k);
-        const double d1 = a * cA[k].x, d2 = b * cA[k].x + a * a * cB[k].x, u = u0[k].x;
+        const double d1 = a * gA[k].x, d2 = b * gA[k].x + a * a * gB[k].x, u = u0[k].x;
         const double v = p.ViscFac * hdif * (d2 + R.or1(k) * d1 - R.or2(k) * u) - p.CorFac * R.ekpump(k) * u;
         impl_out[k] = mk(v, 0.0);
     }
