@@ -1304,6 +1304,9 @@ static void setup(pz_handle *h)
                                       h->sch.l_assembly ? asm_lds_bytes(N) : (size_t)0});
     else need = std::max({need, h->lds_mphase, h->lds_build, h->lds_start, h->lds_inv});
     if (need > lim) throw std::invalid_argument("problem size exceeds the LDS budget of one workgroup");
+    // the integration method's sizes end at n_r 198, as the interface states
+    // (the m-loop's present layout would hold 202)
+    if (!d.coll && !d.fd && N > 198) throw std::invalid_argument("the integration method needs n_r_max <= 198");
     allow_full_lds((int)lim);
     HIPCHK(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
     // device copy of the (now final) descriptor for kernels that read it

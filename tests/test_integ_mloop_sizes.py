@@ -49,3 +49,14 @@ def test_integ_mloop_sizes(n_r, n_cheb, scheme, ra, raxi, buo, pump):
         for f in _fields(cfg):
             err = rel(g.get_field(f), o.get_field(f))
             assert err < max(1e-11, 10 * floors[i][f]), (f, i, err, floors[i][f])
+
+
+@pytest.mark.parametrize("n_r", [199, 202, 203])
+def test_larger_sizes_are_refused(n_r):
+    """The integration method's sizes end at n_r 198 (the largest case above)."""
+    from pizza_amd.config import default_config
+    from pizza_amd.runtime import PizzaError, Run
+    print(f"case: integration n_r {n_r} refused", flush=True)
+    with pytest.raises(PizzaError, match=r"\(-3\)"):
+        Run(default_config(n_r_max=n_r, n_cheb_max=n_r, m_max=6, time_scheme="BPR353", cheb_method="integ",
+                           matrix_solve="direct", radratio=0.35))
