@@ -331,9 +331,11 @@ int pz_ifft(pz_handle *h, const double *spec, double *grid, int n_rad);
  * (n_m, n_r_max) in the layout of pz_get_ddr (m fastest); d_ddf = NULL
  * computes the first derivative only (pz_get_dr).  n_m * n_r_max <= 262144
  * (larger sizes return -2).  Nothing is shared between calls: calls of
- * different handles may overlap, and d_f may be d_df or d_ddf.  Asynchronous
- * on the handle's stream (pz_stream); the caller synchronises before reading
- * d_df.
+ * different handles may overlap, and d_f may be d_df or d_ddf.  Arrays that
+ * overlap in part are taken too, through temporaries of the stream's memory
+ * pool (the one form that allocates); where d_df and d_ddf overlap, d_ddf is
+ * written last.  Asynchronous on the handle's stream (pz_stream); the caller
+ * synchronises before reading d_df.
  */
 int pz_get_ddr_noalloc(pz_handle *h, const double *d_f, double *d_df, double *d_ddf, int n_m,
                        int l_dct_in);

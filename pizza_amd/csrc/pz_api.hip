@@ -2505,7 +2505,12 @@ extern "C" int pz_get_ddr(pz_handle *h, const double *f, double *df, double *ddf
 
 // get_dr / get_ddr on device buffers in the reference layout, read and written
 // there by one kernel with the transforms of pz_get_ddr: no allocation and no
-// memory shared between calls, asynchronous on the handle's stream.
+// memory shared between calls, asynchronous on the handle's stream.  A
+// workgroup reads all rows of its columns before it writes them, so df and ddf
+// may be f.  Arrays that overlap in part would let it overwrite columns that
+// another workgroup has yet to read, or mix the two results: those results go
+// to temporaries of the stream's memory pool and are copied out one after the
+// other, the second last.
 extern "C" int pz_get_ddr_noalloc(pz_handle *h, const double *d_f, double *d_df, double *d_ddf, int n_m,
                                   int l_dct_in)
 {
@@ -2513,11 +2518,30 @@ extern "C" int pz_get_ddr_noalloc(pz_handle *h, const double *d_f, double *d_df,
     const int N = h->N;
     const size_t S = (size_t)n_m * N;
     if (S > PZ_NOALLOC_ELEMS)
-        return fail(h, -2, "pz_get_ddr_noalloc: n_m * n_r_max exceeds the staging limit of 262144 complex values");
+        return fail(h, -2, "pz_get_ddr_noalloc: n_m * n_r_max exceeds 262144 complex values (once a staging limit)");
+    auto partly = [S](const double *a, const double *b) {
+        const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+        return x != y && (x < y ? y - x : x - y) < S * sizeof(cd);
+    };
+    const bool apart = partly(d_f, d_df) || (d_ddf && (partly(d_f, d_ddf) || partly(d_df, d_ddf)));
+    cd *o1 = (cd *)d_df, *o2 = (cd *)d_ddf, *tmp = nullptr;
+    hipError_t e = hipSuccess;
+    if (apart) {
+        e = hipMallocAsync((void **)&tmp, 2 * S * sizeof(cd), h->stream);
+        if (e != hipSuccess) return fail(h, -4, std::string("pz_get_ddr_noalloc: ") + hipGetErrorString(e));
+        o1 = tmp;
+        if (d_ddf) o2 = tmp + S;
+    }
     const int V = dr_ref_vectors(N, n_m), tiles = (n_m + V - 1) / V;
     hipLaunchKernelGGL(k_dr_ref, dim3(8 * ((tiles + 7) / 8)), dim3(256), dr_ref_lds(N, V), h->stream, (const PzDev *)h->ddev,
-                       (const cd *)d_f, (cd *)d_df, (cd *)d_ddf, n_m, l_dct_in, V);
-    hipError_t e = hipGetLastError();
+                       (const cd *)d_f, o1, o2, n_m, l_dct_in, V);
+    e = hipGetLastError();
+    if (apart) {
+        if (e == hipSuccess) e = hipMemcpyAsync(d_df, o1, S * sizeof(cd), hipMemcpyDeviceToDevice, h->stream);
+        if (e == hipSuccess && d_ddf) e = hipMemcpyAsync(d_ddf, o2, S * sizeof(cd), hipMemcpyDeviceToDevice, h->stream);
+        const hipError_t f = hipFreeAsync(tmp, h->stream);
+        if (e == hipSuccess) e = f;
+    }
     if (e != hipSuccess) return fail(h, -4, std::string("pz_get_ddr_noalloc: ") + hipGetErrorString(e));
     return 0;
 }

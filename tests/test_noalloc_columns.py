@@ -3,6 +3,8 @@ columns that a workgroup takes (one, two, four, with a short last group and
 with tiles that do not divide by the eight chiplets), register, Stockham and
 direct-sum transform lengths; written over its own input; and two handles of
 one process at once, whose results must not depend on each other."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -73,3 +75,31 @@ def test_noalloc_two_handles_at_once():
             assert np.array_equal(o.get(f.T.shape).T, v)
         for d in b:
             d.free()
+
+
+@pytest.mark.parametrize("n_r,n_m,at", [(97, 1027, (0, 5, 11)), (33, 700, (700, 0, 33)), (65, 513, (3, 3, 0)), (33, 64, (0, 2112, 31))])
+def test_noalloc_arrays_that_overlap_in_part(n_r, n_m, at):
+    """f, df and ddf at offsets of one buffer, each array overlapping the next
+    in part (or, where offsets are equal, wholly): the derivatives are those
+    of f as it was before the call, ddf written after df."""
+    print(f"case: noalloc derivative, overlapping arrays, n_r {n_r}, {n_m} columns", flush=True)
+    run, hip, S = _run(n_r), _hip(), n_m * n_r
+    f = _field(np.random.default_rng(8), n_m, n_r)
+    buf = _Device(hip, S + max(at))
+    host = np.zeros(S + max(at), dtype=np.complex128)
+    host[at[0]:at[0] + S] = f.T.ravel()
+    buf.put(host)
+    want = host.copy()
+    d1, d2 = run.get_ddr(f, True)
+    want[at[1]:at[1] + S] = d1.T.ravel()
+    want[at[2]:at[2] + S] = d2.T.ravel()
+    assert hip.hipDeviceSynchronize() == 0
+
+    class _At:
+        def __init__(self, o):
+            self.ptr = ctypes.c_void_p(buf.ptr.value + 16 * o)
+
+    _call(run, _At(at[0]), _At(at[1]), _At(at[2]), n_m, 1)
+    assert hip.hipDeviceSynchronize() == 0
+    assert np.array_equal(buf.get(want.shape), want)
+    buf.free()
