@@ -1905,9 +1905,9 @@ static void launch_courant(pz_handle *h)
     hipLaunchKernelGGL(k_courant, dim3(1), dim3(256), 0, h->stream, (const PzDev *)h->ddev);
 }
 
-__global__ void k_force_lmat(PzScheme *s)
+__global__ void k_set_lmat(PzScheme *s, int lMat)
 {
-    if (threadIdx.x == 0) s->lMat = 1;
+    if (threadIdx.x == 0) s->lMat = lMat;
 }
 
 // Stage 1: the matrix rebuild of the run's radial method; the kernels exit
@@ -2047,7 +2047,7 @@ extern "C" int pz_stage_implicit(pz_handle *h, int stage, int lMat)
     if (rc) return rc;
     try {
         if (stage == 1) {
-            if (lMat) hipLaunchKernelGGL(k_force_lmat, dim3(1), dim3(64), 0, h->stream, h->d.ss);
+            if (lMat) hipLaunchKernelGGL(k_set_lmat, dim3(1), dim3(64), 0, h->stream, h->d.ss, 1);
             launch_builds(h);
         }
         launch_implicit(h, stage);
@@ -3013,6 +3013,9 @@ extern "C" int pz_time_kernel(pz_handle *h, int which, int reps, double *avg_ms)
         char *keep = nullptr;
         HIPCHK(hipMalloc(&keep, h->arena_bytes));
         HIPCHK(hipMemcpyAsync(keep, h->arena, h->arena_bytes, hipMemcpyDeviceToDevice, h->stream));
+        // the finite-difference m-loop would rebuild in every repetition if the
+        // last step did: the flag is part of the state that is put back
+        hipLaunchKernelGGL(k_set_lmat, dim3(1), dim3(64), 0, h->stream, h->d.ss, 0);
         hipEvent_t e0, e1;
         HIPCHK(hipEventCreate(&e0));
         HIPCHK(hipEventCreate(&e1));
