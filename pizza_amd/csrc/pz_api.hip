@@ -1251,7 +1251,7 @@ static void setup(pz_handle *h)
     // LDS budgets
     h->lds_radial = (5 * (size_t)h->nm + 7 * (size_t)h->nphi) * sizeof(cd) + 16 * sizeof(double);
     h->mthreads = mloop_threads(N);
-    h->lds_mphase = MpLayout(N, h->mthreads, true, !d.coll && !d.fd).total;
+    h->lds_mphase = mloop_lds(N, h->mthreads, true, !d.coll && !d.fd);
     h->lds_fd = FdLayout(N).total;
     h->lds_fd_loop = FdLoopLayout(N).total;
     h->lds_start = 15 * (size_t)N * sizeof(cd);
@@ -1272,7 +1272,7 @@ static void setup(pz_handle *h)
     h->lds_gj = std::max(gj_lds_bytes<cd>(2 * N), (size_t)1024 * sizeof(double));
     if (d.coll && h->lds_mphase > lim) {
         h->mcoll_l2 = true;
-        h->lds_mphase = MpLayout(N, h->mthreads, false).total;
+        h->lds_mphase = mloop_lds(N, h->mthreads, false);
     }
     if (h->lds_radial > lim) {
         h->radial_big = true;
@@ -3218,8 +3218,8 @@ static void ens_policy(pz_ensemble *e, int policy)
         c.mthreads = (big && (policy & 1) && 2 * c.n <= 256) ? 256 : mloop_threads(c.n);
         c.rad_lds = (big && (policy & 2)) ? 0 : 1;
         // grids whose full layout does not fit read through L2 under any policy
-        if (e->coll && MpLayout(c.n, c.mthreads, true).total > (size_t)lim) c.rad_lds = 0;
-        c.lds_m = MpLayout(c.n, c.mthreads, c.rad_lds != 0).total;
+        if (e->coll && mloop_lds(c.n, c.mthreads, true) > (size_t)lim) c.rad_lds = 0;
+        c.lds_m = mloop_lds(c.n, c.mthreads, c.rad_lds != 0);
         if (c.gexec) { (void)hipGraphExecDestroy(c.gexec); c.gexec = nullptr; }
         if (c.graph) { (void)hipGraphDestroy(c.graph); c.graph = nullptr; }
     }

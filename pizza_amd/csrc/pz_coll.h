@@ -450,7 +450,7 @@ __device__ __forceinline__ void mcoll_body(const PzDev &p, int mi, int istage, i
     const int is = istage - 1;
     const PzScheme *ss = p.ss;
     const int tid = threadIdx.x;
-    const MpLayout lay(N, blockDim.x, RADLDS);
+    const MpLayout lay(N, RADLDS);
     char *lb = (char *)smem;
     cd *V = (cd *)(lb + lay.vec);
     cd *aT = V, *cT = V + N, *eT = V + 2 * N;

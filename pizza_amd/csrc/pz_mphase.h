@@ -112,7 +112,7 @@ __host__ __device__ constexpr int shared_groups(int N, int threads)
 // column groups but the first in registers (matvec_scratch), MatAhead stores
 // those of every group (ahead_scratch), SharedMv [vector][group][n_r rounded
 // up to 4], with half the threads for T and xi and half for psi.
-__host__ __device__ constexpr size_t mloop_scratch(int N, int threads, bool integ)
+constexpr size_t mloop_scratch(int N, int threads, bool integ)
 {
     const size_t ldm = (N + 3) & ~3;
     const size_t need[] = {6 * (2 * (size_t)N - 2) + 16,
@@ -129,14 +129,17 @@ __host__ __device__ constexpr size_t mloop_scratch(int N, int threads, bool inte
     return most;
 }
 
-// LDS layout of k_mphase: working vectors, transform tables and the
-// reduction scratch of the dense solves (16-byte aligned blocks).
+// LDS layout of the m-loop kernels: working vectors, transform tables and, up
+// to the end of the launch's LDS (mloop_lds), the scratch red (16-byte aligned
+// blocks).  The kernels compute the offsets, inlined; the size of red is the
+// host's (computed in the kernels, its list of products takes scratch memory and
+// registers there: fifty BPR353 steps at n_r 97 12.06 ms, 11.73 ms without).
 struct MpLayout {
-    size_t vec = 0, cosT = 0, sinT = 0, rad = 0, red = 0, total = 0;
+    size_t vec = 0, cosT = 0, sinT = 0, rad = 0, red = 0;
     // rad_lds = false: the radial rows and the transform tables stay in
     // global memory (read through L2), which frees PZ_NRADC n_r + 2 L
     // doubles of LDS per workgroup (collocation m-loop only)
-    __host__ __device__ constexpr MpLayout(int N, int threads, bool rad_lds = true, bool integ = false)
+    __host__ __device__ __forceinline__ constexpr MpLayout(int N, bool rad_lds = true)
     {
         size_t o = 0;
         auto take = [&](size_t bytes) { size_t r = o; o += (bytes + 15) & ~(size_t)15; return r; };
@@ -146,10 +149,14 @@ struct MpLayout {
         cosT = rad_lds ? take(sizeof(double) * (2 * L + PZ_NRADC * N)) : 0;
         sinT = cosT + sizeof(double) * L;
         rad = cosT + sizeof(double) * 2 * L;
-        red = take(sizeof(cd) * mloop_scratch(N, threads, integ));
-        total = o;
+        red = o;
     }
 };
+// bytes of LDS that a launch of an m-loop kernel asks for
+constexpr size_t mloop_lds(int N, int threads, bool rad_lds = true, bool integ = false)
+{
+    return MpLayout(N, rad_lds).red + sizeof(cd) * mloop_scratch(N, threads, integ);
+}
 
 
 // The slots of one field at one point that its right-hand side reads: all of
@@ -476,7 +483,7 @@ __device__ __forceinline__ void mphase_body(const PzDev &p, int mi, int istage, 
     const int is = istage - 1;
     const PzScheme *ss = p.ss;
     const int tid = threadIdx.x;
-    const MpLayout lay(N, blockDim.x, true, true);
+    const MpLayout lay(N);
     char *lb = (char *)smem;
     cd *V = (cd *)(lb + lay.vec);
     // e and a of a field are adjacent: the 2 n_r inputs of its explicit assembly

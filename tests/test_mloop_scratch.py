@@ -42,8 +42,7 @@ constexpr size_t shared_top(int N, int nt, int nvec)
 }
 constexpr size_t allotted(int N, int nt, bool rad, bool integ)
 {
-    const MpLayout l(N, nt, rad, integ);
-    return (l.total - l.red) / sizeof(cd);
+    return (mloop_lds(N, nt, rad, integ) - MpLayout(N, rad).red) / sizeof(cd);
 }
 // the first n_r of [lo, hi] whose products leave the scratch; 0: none
 constexpr int collocation(int lo, int hi, bool rad, bool narrow)
