@@ -84,8 +84,14 @@ __device__ __forceinline__ void lds_store(cd *q, int i, cd v)
 // waits for every outstanding global load and store of the wave, which keeps
 // a phase's result stores (one to two microseconds) and loads issued ahead of
 // their use on the chain; between phases that exchange values through LDS
-// alone nothing needs them.  Where another thread reads global memory written
-// before the barrier, __syncthreads stays.
+// alone nothing needs them.  For the m-loop kernels, which load ahead, the
+// transforms and products that they call (fft_stockham, dct_fft, dr_fft,
+// block_matvec) and the stages of the in-place transforms (1 % of a
+// finite-difference gradient, whose transposed radial loop parks a grid in
+// global memory): these order no global memory, so a caller that passes global
+// memory from thread to thread has a __syncthreads of its own.  Elsewhere it
+// gains nothing (radial loops, reductions and the finite-difference m-loop:
+// 0.99x to 1.01x), and __syncthreads stays.
 __device__ __forceinline__ void lds_barrier()
 {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -656,12 +662,12 @@ __device__ double block_reduce(double v, double *scratch, int op /*0 sum, 1 max*
         double u = __shfl_xor(v, o, 64);
         v = op == 0 ? v + u : fmax(v, u);
     }
-    lds_barrier();
+    __syncthreads();
     if (lane == 0) scratch[w] = v;
-    lds_barrier();
+    __syncthreads();
     double r = scratch[0];
     for (int i = 1; i < nw; i++) r = op == 0 ? r + scratch[i] : fmax(r, scratch[i]);
-    lds_barrier();
+    __syncthreads();
     return r;
 }
 
@@ -880,9 +886,10 @@ __device__ __forceinline__ void courant_decide(const PzDev &p, double dtr, doubl
 // below holds the count until the workgroup's own atomics have been performed,
 // which is what a device-scope release waits for too.  Written as an
 // acquire-release count the same line also writes the L2 back and invalidates
-// it, in every workgroup: 1.1 us (ARS222, n_r 49) to 4.4 us (BPR353, n_r 97) a
-// step, 0.97x to 0.99x on whole runs; nothing but these three words, which only
-// atomics touch, passes between the workgroups.  Positive doubles compare like
+// it in every workgroup: nothing up to n_r 129, but 4 to 6 us a step at n_r 257
+// with 683 modes (fifty SBDF3 steps 10.43 ms, then 10.64 to 10.75 ms in three
+// comparisons).  Nothing but these three words, which only atomics touch,
+// passes between the workgroups.  Positive doubles compare like
 // their bit patterns, so the limits are those of k_courant.  Saves a launch of
 // one workgroup, 4.5 to 7.3 us of a step.  lds: 8 doubles.
 __device__ __forceinline__ void courant_tail(const PzDev &p, double dtrk, double dthk, double *lds)
@@ -934,7 +941,7 @@ __device__ __forceinline__ void radial_loop_body(const PzDev &p, int nr, int is,
         spec[3 * nm + i] = p.l_heat ? p.temp[q] : mk(0, 0);
         spec[4 * nm + i] = p.l_chem ? p.xi[q] : mk(0, 0);
     }
-    lds_barrier();
+    __syncthreads();
     // Reynolds-stress m-sum (radial_loop.f90:267-278)
     double part = 0.0;
     for (int i = threadIdx.x; i < nm; i += blockDim.x) {
@@ -961,14 +968,14 @@ __device__ __forceinline__ void radial_loop_body(const PzDev &p, int nr, int is,
     if (Pw) {
         fft_wave_phi(Pw, nin, packed, [=](int tr, int k, cd v) { bufb[tr * n + k] = v; },
                      [=](int k) { const cd w = twl[k]; return mk(w.x, -w.y); });
-        lds_barrier();
+        __syncthreads();
         g = bufb;
     } else {
         for (int t = threadIdx.x; t < nin * n; t += blockDim.x) {
             const int tr = t / n;
             bufa[t] = packed(tr, t - tr * n);
         }
-        lds_barrier();
+        __syncthreads();
         g = fft_stockham(bufa, bufb, n, nin, +1, p.radices, p.nrad,
                          [&](int k) { const cd w = twl[k]; return mk(w.x, -w.y); });
     }
@@ -1007,13 +1014,13 @@ __device__ __forceinline__ void radial_loop_body(const PzDev &p, int nr, int is,
             o[(p.l_heat ? 2 : 1) * n + j] = mk(up * X, rr * us * X);
         }
     }
-    lds_barrier();
+    __syncthreads();
     cd *other = (o == bufa) ? bufb : bufa;
     cd *Z;
     if (Pw) {
         fft_wave_phi(Pw, nout, [=](int tr, int i) { return o[tr * n + i]; },
                      [=](int tr, int k, cd v) { other[tr * n + k] = v; }, [=](int k) { return twl[k]; });
-        lds_barrier();
+        __syncthreads();
         Z = other;
     } else {
         Z = fft_stockham(o, other, n, nout, -1, p.radices, p.nrad, [&](int k) { return twl[k]; });
@@ -1095,21 +1102,21 @@ __device__ __forceinline__ void radial_loop_big_body(const PzDev &p, int nr, int
         }
         (tr == 0 ? s0 : (tr == 1 ? s1 : s2))[k] = z;
     }
-    lds_barrier();
+    __syncthreads();
     // one complex FFT at a time; the result lands in the column or in the
     // scratch, whose roles are then exchanged
     {
         cd *g = fft_stockham(s0, sc, n, 1, +1, p.radices, p.nrad, bwd);
         if (g != s0) { sc = s0; s0 = g; }
-        lds_barrier();
+        __syncthreads();
         g = fft_stockham(s1, sc, n, 1, +1, p.radices, p.nrad, bwd);
         if (g != s1) { sc = s1; s1 = g; }
         if (p.l_chem) {
-            lds_barrier();
+            __syncthreads();
             g = fft_stockham(s2, sc, n, 1, +1, p.radices, p.nrad, bwd);
             if (g != s2) { sc = s2; s2 = g; }
         }
-        lds_barrier();
+        __syncthreads();
     }
     double dtrk = 1.0e10, dthk = 1.0e10; // thread 0
     if (courant) {
@@ -1141,21 +1148,21 @@ __device__ __forceinline__ void radial_loop_big_body(const PzDev &p, int nr, int
         s1[j] = mk(up * T, rr * us * T);
         if (p.l_chem) s2[j] = mk(up * X, rr * us * X);
     }
-    lds_barrier();
+    __syncthreads();
     {
         cd *g = fft_stockham(s0, sc, n, 1, -1, p.radices, p.nrad, fwd);
         if (g != s0) { sc = s0; s0 = g; }
         if (p.l_heat) {
-            lds_barrier();
+            __syncthreads();
             g = fft_stockham(s1, sc, n, 1, -1, p.radices, p.nrad, fwd);
             if (g != s1) { sc = s1; s1 = g; }
         }
         if (p.l_chem) {
-            lds_barrier();
+            __syncthreads();
             g = fft_stockham(s2, sc, n, 1, -1, p.radices, p.nrad, fwd);
             if (g != s2) { sc = s2; s2 = g; }
         }
-        lds_barrier();
+        __syncthreads();
     }
     // unpack, normalise and post-scale (radial_loop.f90:350-386)
     const double or1 = p.or1[nr];
@@ -1240,7 +1247,7 @@ __device__ __forceinline__ void radial_loop_inplace_body(const PzDev &p, int nr,
     }
     for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
     if ((threadIdx.x & 63) == 0) msr[threadIdx.x >> 6] = part;
-    lds_barrier();
+    __syncthreads();
     fft_inplace(s0, n, 2, +1, p.radices, p.nrad, bwd, om);
     double dtrk = 1.0e10, dthk = 1.0e10; // thread 0
     if (courant) {
@@ -1270,7 +1277,7 @@ __device__ __forceinline__ void radial_loop_inplace_body(const PzDev &p, int nr,
         s0[j] = mk(up * om, rr * us * om);
         s1[j] = mk(up * T, rr * us * T);
     }
-    lds_barrier();
+    __syncthreads();
     fft_inplace(s0, n, p.l_heat ? 2 : 1, -1, p.radices, p.nrad, fwd, om);
     // unpack, normalise and post-scale (radial_loop.f90:350-386)
     const double or1 = p.or1[nr];

@@ -693,7 +693,7 @@ __device__ __forceinline__ void fd_mloop_body(const PzDev &p, int mi, int istage
         if (m == 0) { gP[0] = z; gP[N + 1] = z; }
         else { gP[0] = z; gP[1] = z; gP[N + 2] = z; gP[N + 3] = z; }
     }
-    lds_barrier();
+    __syncthreads();
     // the solves, one wave each (blocks of 256 threads)
     const int wave = tid >> 6;
     if (wave == 0 && hT) fd_tri_solve_wave(N, mT, mT + N, mT + 2 * N, gT);
@@ -702,13 +702,13 @@ __device__ __forceinline__ void fd_mloop_body(const PzDev &p, int mi, int istage
         if (m == 0) fd_tri_solve_wave(N, (const double *)mP, (const double *)mP + N, (const double *)mP + 2 * N, gP);
         else fd_penta_solve_wave(N, mP, mP + N, mP + 2 * N, mP + 3 * N, mP + 4 * N, gP);
     }
-    lds_barrier();
+    __syncthreads();
     if (tid == 0) {
         if (hT) fd_ghost_scalar(gT, N, p.ktopt, p.kbott, R, fd_wall(p, p.topt, mi), fd_wall(p, p.bott, mi));
         if (hX) fd_ghost_scalar(gX, N, p.ktopxi, p.kbotxi, R, fd_wall(p, p.topxi, mi), fd_wall(p, p.botxi, mi));
         fd_ghost_psi(p, R, m, gP);
     }
-    lds_barrier();
+    __syncthreads();
     const int inext = (istage == p.nstages) ? 1 : istage + 1;
     // implicit terms for the next stage; also before a CNAB2 start-up step
     const int lcalc = p.l_imp_calc_rhs[inext - 1] || (p.bridge && ss->n_steps + 1 <= p.nold - 1);
