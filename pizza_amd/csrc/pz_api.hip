@@ -8,7 +8,6 @@
 #include <cstdlib>
 #include <cstdio>
 #include <cstring>
-#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -593,8 +592,9 @@ static std::vector<double> rhs_band(const pz_handle *h, int K, int nbounds, cons
 }
 
 // The m-independent linear maps of the integration m-loop, composed in long
-// double from the bands (T_RHSE1, P_RHSE1, P_RHSE2, P_RHSE3), costf (with and
-// without the modes above n_cheb) and the radial derivative.  All of them
+// double from the bands of the explicit terms (T and xi bT; psi bP, at m = 0
+// bP0) and of the buoyancy (bB), costf (with and without the modes above
+// n_cheb) and the radial derivative.  All of them
 // follow from the cosine table in O(n_r^2): the derivative of Chebyshev
 // coefficients is a sum over every second higher one, and costf g costf of a
 // radial function g a sum of two cosine coefficients of g.
@@ -677,17 +677,13 @@ static void build_operators(pz_handle *h)
     };
     // m-independent RHS bands
     {
-        auto s = rows(3, {&L.I2R1}, {1});
-        h->d.T_RHSE1 = h->upload(rhs_band(h, 3, 2, s.data()));
-        s = rows(4, {&L.I2R2}, {1});
-        h->d.T_RHSE2 = h->upload(rhs_band(h, 4, 2, s.data()));
-        h->d.P_RHSE1 = h->upload(rhs_band(h, 4, 2, s.data()));
-        s = rows(8, {&L.I4R4}, {1});
-        h->d.P_RHSE2 = h->upload(rhs_band(h, 8, 4, s.data()));
-        s = rows(7, {&L.I4R3}, {1});
-        h->d.P_RHSE3 = h->upload(rhs_band(h, 7, 4, s.data()));
-        compose_operators(h, rhs_band(h, 3, 2, rows(3, {&L.I2R1}, {1}).data()), rhs_band(h, 4, 2, rows(4, {&L.I2R2}, {1}).data()),
-                          rhs_band(h, 8, 4, rows(8, {&L.I4R4}, {1}).data()), rhs_band(h, 7, 4, s.data()));
+        const std::vector<double> T1 = rhs_band(h, 3, 2, rows(3, {&L.I2R1}, {1}).data());
+        const std::vector<double> P1 = rhs_band(h, 4, 2, rows(4, {&L.I2R2}, {1}).data());
+        const std::vector<double> P2 = rhs_band(h, 8, 4, rows(8, {&L.I4R4}, {1}).data());
+        const std::vector<double> P3 = rhs_band(h, 7, 4, rows(7, {&L.I4R3}, {1}).data());
+        h->d.T_RHSE2 = h->upload(P1); // old slots of T and xi: the same stencil, I2 r^2
+        h->d.P_RHSE2 = h->upload(P2);
+        compose_operators(h, T1, P1, P2, P3);
     }
     std::vector<double> TRHSI((size_t)nm * N * 5, 0.0), PRHSI((size_t)nm * N * 17, 0.0);
     std::vector<double2> PRHSIL((size_t)nm * N * 17, make_double2(0, 0));
@@ -887,7 +883,8 @@ static void allow_full_lds(int lim)
                              (const void *)k_start, (const void *)k_build_inv, (const void *)k_mcoll,
                              (const void *)k_start_coll, (const void *)k_dr_ref, (const void *)k_build_lhs_batch,
                              (const void *)k_mphase_batch, (const void *)k_mphase_batch_small, (const void *)k_radial_loop_batch,
-                             (const void *)k_build_inv_batch, (const void *)k_mcoll_batch<true>, (const void *)k_mcoll_batch<false>,                              (const void *)k_fd_mloop, (const void *)k_fd_start, (const void *)k_radial_loop_big,
+                             (const void *)k_build_inv_batch, (const void *)k_mcoll_batch<true>, (const void *)k_mcoll_batch<false>,
+                             (const void *)k_fd_mloop, (const void *)k_fd_start, (const void *)k_radial_loop_big,
                              (const void *)k_radial_loop_inplace,
                              (const void *)k_adj_probe, (const void *)k_mcoll_adj, (const void *)k_radial_adj,
                              (const void *)k_start_coll_adj, (const void *)k_assemble_coll,

@@ -366,7 +366,7 @@ __global__ void __launch_bounds__(256) k_assemble_fd(const PzDev *__restrict__ p
     cd *gT = (cd *)(lb + lay.gT), *gX = (cd *)(lb + lay.gX), *gP = (cd *)(lb + lay.gP);
     cd *V = (cd *)(lb + lay.vec);
     cd *aT = V, *aX = V + N, *aP = V + 2 * N, *usv = V + 3 * N, *Tv = V + 4 * N, *Xv = V + 5 * N;
-    double *eD = (double *)(lb + lay.mT), *eL = eD + N, *eU = eD + 2 * N;
+    double *eD = (double *)(lb + lay.mE), *eL = eD + N, *eU = eD + 2 * N;
     const bool hT = p.l_heat, hX = p.l_chem;
     const RadView R(p.radc, N);
     const FdView S(p.fdc, N);

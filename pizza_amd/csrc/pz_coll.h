@@ -7,8 +7,6 @@
 #include "pz_mphase.h"
 #include "pz_gj.h"
 
-__device__ __forceinline__ double msub(double a, double b) { return a - b; }
-__device__ __forceinline__ cd msub(cd a, cd b) { return csub(a, b); }
 // modulus (Fortran abs of a real or complex element)
 __device__ __forceinline__ double mabs2(double a) { return fabs(a); }
 __device__ __forceinline__ double mabs2(cd a) { return hypot(a.x, a.y); }

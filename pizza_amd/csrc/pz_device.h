@@ -1567,7 +1567,8 @@ __device__ void wave_gbtrs_fast(int n, const M *ab, int ld, const int *ipiv, con
     }
 }
 
-// bordered solve with all factors in LDS
+// bordered solve (algebra_lapack.f90:332-416) by one wave, rhs and all factors
+// in LDS
 template <class M, int KL, int KU>
 __device__ void wave_bordered_fast(int N, int nt, const M *A1, const int *p1, const M *A2, const M *A3,
                                    const M *A4, const int *p4, const M *dinv, cd *rhs)
@@ -1576,40 +1577,6 @@ __device__ void wave_bordered_fast(int N, int nt, const M *A1, const int *p1, co
     const int nb = N - nt, ld = 2 * KL + KU + 1;
     cd *r2 = rhs + nt;
     wave_gbtrs_fast<M, KL, KU>(nb, A4, ld, p4, dinv, r2);
-    for (int i = 0; i < nt; i++) {
-        double sx = 0.0, sy = 0.0;
-        for (int c = lane; c < nb; c += 64) {
-            cd t = mmul(A2[i + (size_t)c * nt], r2[c]);
-            sx += t.x;
-            sy += t.y;
-        }
-        sx = wave_sum(sx);
-        sy = wave_sum(sy);
-        if (lane == 0) rhs[i] = mk(rhs[i].x - sx, rhs[i].y - sy);
-    }
-    __builtin_amdgcn_wave_barrier();
-    if (lane == 0) small_getrs<M>(nt, A1, p1, rhs);
-    __builtin_amdgcn_wave_barrier();
-    cd y[4];
-    for (int c = 0; c < nt; c++) y[c] = rhs[c];
-    for (int i = lane; i < nb; i += 64) {
-        cd v = r2[i];
-        for (int c = 0; c < nt; c++) v = csub(v, mmul(A3[i + (size_t)c * nb], y[c]));
-        r2[i] = v;
-    }
-    __builtin_amdgcn_wave_barrier();
-}
-
-// bordered solve (algebra_lapack.f90:332-416) by one wave; rhs in LDS
-template <class M>
-__device__ void wave_bordered_solve(int N, int nt, int kl, int ku, int ld, const M *A1, const int *p1,
-                                    const M *A2, const M *A3, const M *A4, const int *p4, cd *rhs)
-{
-    const int lane = threadIdx.x & 63;
-    const int nb = N - nt;
-    cd *r2 = rhs + nt;
-    wave_gbtrs<M>(nb, kl, ku, A4, ld, p4, r2);
-    // rhs1 <- rhs1 - A2 r2
     for (int i = 0; i < nt; i++) {
         double sx = 0.0, sy = 0.0;
         for (int c = lane; c < nb; c += 64) {

@@ -260,12 +260,12 @@ __device__ __forceinline__ void fd_lu5_scale(int N, const cd *d, cd *l1, cd *l2,
     }
 }
 
-// LDS layout of the start, rebuild and assembly kernels of the
-// finite-difference method (16-byte blocks): ghosted columns gT, gX
-// (N + 2), gP (N + 4; u_phi of m = 0 at offset 1), six N-vectors, then the
-// factorised systems of this m.
+// LDS layout of the start and assembly kernels of the finite-difference
+// method (16-byte blocks): ghosted columns gT, gX (N + 2), gP (N + 4; u_phi of
+// m = 0 at offset 1), six N-vectors, then the tridiagonal system of the
+// assembly (3 N doubles).
 struct FdLayout {
-    size_t gT, gX, gP, vec, mT, mX, mP, total;
+    size_t gT, gX, gP, vec, mE, total;
     __host__ __device__ FdLayout(int N)
     {
         size_t o = 0;
@@ -274,9 +274,7 @@ struct FdLayout {
         gX = take(sizeof(cd) * (N + 2));
         gP = take(sizeof(cd) * (N + 4));
         vec = take(sizeof(cd) * 6 * (size_t)N);
-        mT = take(sizeof(double) * 3 * (size_t)N);
-        mX = take(sizeof(double) * 3 * (size_t)N);
-        mP = take(sizeof(cd) * 5 * (size_t)N);
+        mE = take(sizeof(double) * 3 * (size_t)N);
         total = o;
     }
 };

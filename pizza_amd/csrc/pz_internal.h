@@ -100,10 +100,9 @@ struct PzDev {
 
     // m-independent RHS bands, row-major [n_r][2K+1] in column-offset order
     // (entry K+d is column i+d), already multiplied by rnorm
-    const double *T_RHSE1, *T_RHSE2;           // K = 3, 4
-    const double *P_RHSE1, *P_RHSE2, *P_RHSE3; // K = 4, 8, 7
+    const double *T_RHSE2, *P_RHSE2; // K = 4, 8
     // m-independent maps of the integration m-loop composed from the
-    // transforms, the radial derivative and those bands, column-major
+    // transforms, the radial derivative and such bands, column-major
     // [col][n_r rounded up to 4]: [band costf | -band costf d/dr] of the explicit assembly of
     // T and xi (T_M) and of psi (P_M; m = 0: P_M0, band costf alone), 2 n_r
     // (n_r) columns, and the implicit buoyancy's band costf (-rgrav / r)
