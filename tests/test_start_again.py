@@ -31,3 +31,52 @@ def test_start_again(method, scheme):
     a, b = go(again, 1.0e-3, 5), go(new, 1.0e-3, 5)
     for x, y in zip(a, b):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("method,scheme", [("integ", "SBDF3"), ("colloc", "SBDF3"), ("fd", "SBDF2")])
+def test_restart_behind_a_captured_step(method, scheme, tmp_path):
+    """A handle that has stepped reads checkpoints and starts from them: one of
+    its own run (the history continues, no CNAB2 start-up steps), one of a run
+    with another Ekman number and fewer slots (start-up steps, a first
+    Adams-Bashforth step), and a fresh start again.  Each time it goes on as a
+    new handle does, bit for bit: the start-up flag in the descriptor and the
+    scheme state change under the captured step."""
+    from pizza_amd import workloads as W
+    from pizza_amd.config import default_config
+    from pizza_amd.runtime import Run
+    kw = dict(radial_scheme="FD") if method == "fd" else dict(cheb_method=method, matrix_solve="direct")
+    kw.update(n_r_max=33, n_cheb_max=33, m_max=8, dtMax=1.0e-6, ra=1.0e6, raxi=1.0e6, sc=3.0, pr=1.0, radratio=0.35)
+    cfg, other = default_config(time_scheme=scheme, ek=1.0e-4, **kw), default_config(time_scheme="CNAB2", ek=2.0e-4, **kw)
+    print(f"case: restarts behind a captured step, {method} {scheme}", flush=True)
+
+    def fresh(r, c):
+        for f in ("us", "up", "om", "psi"):
+            r.set_field(f, np.zeros((r.n_m, 33), complex))
+        W.seed_run(r, c, amp_t=1.0e-3, amp_xi=1.0e-3)
+        r.start()
+        r.step(6)
+
+    def restart(r, path):
+        r.read_checkpoint(path)
+        r.start()
+        r.step(5)
+
+    def same(a, b):
+        assert a.time() == b.time()
+        for f in ("temp", "xi", "us", "up", "om"):
+            assert np.array_equal(a.get_field(f), b.get_field(f)), f
+
+    run, donor = Run(cfg), Run(other)
+    fresh(run, cfg)
+    fresh(donor, other)
+    run.write_checkpoint(tmp_path / "own")
+    donor.write_checkpoint(tmp_path / "other")
+    for name in ("own", "other", "own"):
+        new = Run(cfg)
+        restart(run, tmp_path / name)
+        restart(new, tmp_path / name)
+        same(run, new)
+    new = Run(cfg)
+    fresh(run, cfg)
+    fresh(new, cfg)
+    same(run, new)
