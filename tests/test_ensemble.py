@@ -123,3 +123,13 @@ def test_ensemble_members_match_oracle_over_500_steps():
         for f in FIELDS:
             err = rel(r.get_field(f), o.get_field(f))
             assert err < 1e-8, (k, f, err)
+
+
+@pytest.mark.parametrize("sizes", [((97, 32), (66, 24), (97, 48)), ((33, 16), (97, 16), (129, 24))])
+def test_larger_integration_ensembles_equal_single_runs(sizes):
+    """Classes above n_r 65 (the 512-thread form of the batched m-loop), alone
+    and beside one of the small form, bitwise against the single runs."""
+    from pizza_amd import workloads as W
+    cfgs = [W.small_bpr353(n_r, m) for n_r, m in sizes]
+    cfgs[1].ra = 1.0e7
+    _check_equal(cfgs, lambda r, c, k: W.seed_run(r, c, seed=W.SEED + k), 4)
