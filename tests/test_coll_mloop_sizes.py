@@ -3,13 +3,17 @@ ahead, its thread groups and its tables take another form: fewer rows than
 columns loaded ahead (8 to 13 and 16, 17), one and several rows a thread,
 register and Stockham FFTs, tables in LDS and in L2 (n_r 97 and 256); T alone,
 xi alone and both; every slot of SBDF4 and the stage sums of ARS443; the
-coupled and the influence-matrix solve.  One and six steps against the oracle, each
-field within ten times what one rounding of dt moves the oracle's own result
-(its conditioning), and at least 1e-11; above n_r 97 that grows as n_r^4, as
-the condition of the second-derivative collocation matrices does, whose
-inverses two implementations round differently (n_r 256: 4.9e-10), and there
-one step is compared, since the difference of an explicit inverse from an LU
-solve grows with each step at that condition."""
+coupled and the influence-matrix solve.  One and six steps against the oracle,
+each field within ten times what one rounding of the initial state moves the
+oracle's own result (its conditioning), and at least 1e-11; above n_r 97 that
+grows as n_r^4 in the first step, as the condition of the second-derivative
+collocation matrices does, whose inverses two implementations round
+differently (n_r 256: 4.9e-10).  In each further step the residual of an
+explicit inverse, which an LU solve does not leave, comes in once more, so the
+difference grows in proportion to the steps: at n_r 256 the elimination with
+row swaps that this one replaced was 2.3e-9, 1.0e-8 and 1.8e-8 away after two,
+four and six steps (u_phi; 2.0e-9, 6.0e-9 and 1.1e-8 with this one), and the
+bound for six steps is four times its 1.8e-8."""
 import pytest
 
 from helpers import rel
@@ -50,9 +54,10 @@ def test_coll_mloop_sizes(n_r, scheme, ra, raxi, buo, pump, solve):
     for x in (g, o):
         seed(x)
         x.start()
-    for i, n in enumerate((1, 5) if n_r <= 97 else (1,)):
+    least = (1e-11, 1e-11) if n_r <= 97 else (1e-11 * (n_r / 97) ** 4, 7.2e-8)
+    for i, n in enumerate((1, 5)):
         g.step(n)
         o.step(n)
         for f in _fields(cfg):
             err = rel(g.get_field(f), o.get_field(f))
-            assert err < max(1e-11 * max(1.0, n_r / 97) ** 4, 10 * floors[i][f]), (f, i, err, floors[i][f])
+            assert err < max(least[i], 10 * floors[i][f]), (f, i, err, floors[i][f])

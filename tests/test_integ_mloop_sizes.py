@@ -4,8 +4,9 @@ smallest n_r, both thread counts (n_r 65 and 66), register FFTs (33, 97) and
 Stockham FFTs, both limits of the column groups (160 and 161), the largest
 n_r; fewer Chebyshev modes than radii; T alone, xi alone and both; implicit
 and explicit buoyancy; every slot of SBDF4 and the stage sums of ARS443.
-Two steps against the oracle, each field within ten times what one rounding
-of dt moves the oracle's own result (its conditioning), and at least 1e-11."""
+One and six steps against the oracle, each field within ten times what one
+rounding of the initial state moves the oracle's own result (its conditioning),
+and at least 1e-11."""
 import pytest
 
 from helpers import rel
