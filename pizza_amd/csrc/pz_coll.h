@@ -180,8 +180,8 @@ __device__ void coll_assemble(const PzDev &p, const RadView &R, int fld, int m, 
 }
 
 // get_omMat / get_psiMat of the influence-matrix method
-// (update_psi_coll_dmat.f90:829-983) into W (row-major, N x N): which = 0 the omega operator (identity minus the implicit
-// viscous term), 1 the stream-function operator with beta; zero rows at
+// (update_psi_coll_dmat.f90:829-983) into W (row-major, N x N): which = 0 the
+// omega operator (identity minus the implicit viscous term), 1 the stream-function operator with beta; zero rows at
 // both walls, boundary_fac on the first and last columns, then the row
 // (fac[0..N)) and column (fac[N..2N)) max-scalings
 __device__ void coll_assemble_dmat(const PzDev &p, const RadView &R, int which, int m, double hdif, double *W,
@@ -436,7 +436,7 @@ __device__ __forceinline__ void coll_uphi0_impl(const PzDev &p, const RadView &R
 // order LDS only, and a single run has the first PFS and PFP columns of its
 // inverses in registers long before their products (0: none, for batches,
 // whose workgroups share a CU within 128 registers; the sums are the same).
-// Measured a launch: 48.3 us at n_r 129 and 171 modes (51.8 with loads where
+// Measured a launch: 47.6 us at n_r 129 and 171 modes (51.8 with loads where
 // they were used), 35.1 us a stage of ARS222 at n_r 49 and 49 modes (37.4),
 // 20.8 us at n_r 33 and 33 modes (23.1).
 template <bool RADLDS, int PFS, int PFP>

@@ -473,7 +473,7 @@ __device__ __forceinline__ void mphase_psi_at(const PzDev &p, const RadView &R, 
 // behind the inputs, long before their use, the slots of a multistep scheme
 // rotate from the values the right-hand side reads, and everything behind
 // the psi solve (up to five transforms, six bands) is one phase.  Measured at
-// n_r 97, 129 modes, both scalars: 32.5 us a launch (42.7 us before).
+// n_r 97, 129 modes, both scalars: 31.9 us a launch (42.7 us before).
 template <int PFS, int PFP, int U>
 __device__ __forceinline__ void mphase_body(const PzDev &p, int mi, int istage, int exp_calc)
 {
@@ -844,8 +844,8 @@ __global__ void __launch_bounds__(PZ_MPHASE_THREADS) k_mphase_batch(PzBatch b, i
     mphase_body<10, 16, 8>(*b.runs[e.x], e.y, istage, exp_calc);
 }
 // n_r <= 65 (256 threads): fewer columns ahead and 168 registers, so that
-// three workgroups of many small runs share a CU (48 runs at n_r 33: 199 us a
-// step with the larger form); the sums are the same
+// three workgroups of many small runs share a CU (48 runs at n_r 33: 179 us a
+// step, 199 us with the larger form); the sums are the same
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) k_mphase_batch_small(PzBatch b, int istage, int exp_calc)
 {
     const int2 e = b.map[blockIdx.x];
