@@ -103,3 +103,40 @@ def test_noalloc_arrays_that_overlap_in_part(n_r, n_m, at):
     assert hip.hipDeviceSynchronize() == 0
     assert np.array_equal(buf.get(want.shape), want)
     buf.free()
+
+
+@pytest.mark.parametrize("at", [(0, 4000, 8000), (0, 5, 11)])
+def test_noalloc_under_capture(at):
+    """The call captured on the handle's stream and replayed with other inputs,
+    eager work between the replays: arrays apart (one kernel) and arrays that
+    overlap in part (temporaries, copies)."""
+    print(f"case: noalloc derivative captured, offsets {at}", flush=True)
+    n_r, n_m = 33, 100
+    run, hip, S = _run(n_r), _hip(), n_m * n_r
+    stream = ctypes.c_void_p(run.stream())
+    buf, rng = _Device(hip, S + max(at)), np.random.default_rng(9)
+
+    class _At:
+        def __init__(self, o):
+            self.ptr = ctypes.c_void_p(buf.ptr.value + 16 * o)
+
+    graph, ex = ctypes.c_void_p(), ctypes.c_void_p()
+    assert hip.hipStreamBeginCapture(stream, 1) == 0  # thread-local
+    _call(run, _At(at[0]), _At(at[1]), _At(at[2]), n_m, 1)
+    assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(4):
+        f = _field(rng, n_m, n_r)
+        host = np.zeros(S + max(at), dtype=np.complex128)
+        host[at[0]:at[0] + S] = f.T.ravel()
+        want = host.copy()
+        d1, d2 = run.get_ddr(f, True)  # eager work of the same handle
+        want[at[1]:at[1] + S] = d1.T.ravel()
+        want[at[2]:at[2] + S] = d2.T.ravel()
+        buf.put(host)
+        assert hip.hipDeviceSynchronize() == 0
+        assert hip.hipGraphLaunch(ex, stream) == 0
+        assert hip.hipDeviceSynchronize() == 0
+        assert np.array_equal(buf.get(want.shape), want)
+    assert hip.hipGraphExecDestroy(ex) == 0 and hip.hipGraphDestroy(graph) == 0
+    buf.free()
